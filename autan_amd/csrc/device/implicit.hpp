@@ -19,8 +19,8 @@
 //                             the cells (an exact minimum of the FP64 values);
 // and the GCR's vector updates (solvers/src/gcr.cpp). Everything in FP64, no contraction, so every
 // value equals the host restatement's. Layouts (chosen for the relaxation, which streams a colour's
-// rows): the rows are numbered by position in the colour-major cell order (the cells of colour 0
-// ascending, then colour 1's, ...); the diagonal and inverse blocks are 25 contiguous values per
+// rows): the rows are numbered by position in the colour by colour cell order (colour 0's cells,
+// then colour 1's, ..., in each those with a neighbour of a higher colour first); the diagonal and inverse blocks are 25 contiguous values per
 // position; a row's off-diagonal blocks are its entries, 25 contiguous values each, so a colour's
 // rows and blocks are one contiguous run; the solve's vectors (the right-hand side, du, the GCR's
 // directions) hold a cell's five values together, value q of cell c at 5 c + q.
@@ -277,6 +277,28 @@ __global__ __launch_bounds__(kBlock) void k_impl_relax(ImplRows rows, int first,
   const int t = (blockIdx.x * (kBlock / kWave) + static_cast<int>(threadIdx.x / kWave)) * kRelaxGroups + g;
   const bool active = g < kRelaxGroups && t < count;
   impl_relax_rows(rows, first + t, active, offd, inverse, b, x);
+}
+
+// The first relaxation of the sweeps from x = 0, colour 0's `count` rows (positions 0 .. count):
+// x_c = D_c^-1 b_c, every neighbour's value being zero, without reading an off-diagonal block;
+// and x = 0 on the other rows up to n. The blocks are finite here (each is a term of a diagonal
+// block, and an inverse met a non-finite pivot otherwise and the solve was refused), so the products
+// left out are zeros; a zero's sign in b_c - 0 is lost in the inverse's product, whose sum starts at
+// +0.
+__global__ __launch_bounds__(kBlock) void k_impl_relax_start(ImplRows rows, int count, int n,
+                                                             const double* __restrict__ inverse,
+                                                             const double* __restrict__ b, double* __restrict__ x) {
+  int q;
+  const int p = impl_group_item(q);
+  if (p < 0 || p >= n) return;
+  const long long c = rows.cell[p];
+  double s = 0.0;
+  if (p < count) {
+    const double* ip = inverse + 25LL * p + 5 * q;
+#pragma unroll
+    for (int j = 0; j < 5; ++j) s += ip[j] * b[5 * c + j];
+  }
+  x[5 * c + q] = s;
 }
 
 // Launch width of k_impl_relax for `count` cells.
