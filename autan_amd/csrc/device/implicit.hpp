@@ -19,11 +19,14 @@
 //                             the cells (an exact minimum of the FP64 values);
 // and the GCR's vector updates (solvers/src/gcr.cpp). Everything in FP64, no contraction, so every
 // value equals the host restatement's. Layouts (chosen for the relaxation, which streams a colour's
-// rows): the rows are numbered by position in the colour by colour cell order (colour 0's cells,
-// then colour 1's, ..., in each those with a neighbour of a higher colour first); the diagonal and inverse blocks are 25 contiguous values per
-// position; a row's off-diagonal blocks are its entries, 25 contiguous values each, so a colour's
-// rows and blocks are one contiguous run; the solve's vectors (the right-hand side, du, the GCR's
-// directions) hold a cell's five values together, value q of cell c at 5 c + q.
+// rows): the rows are numbered by position, colour by colour, in each colour those with a neighbour of
+// a higher colour first; each of these groups is cut into slices of kSlice = 12 rows (the last padded
+// with empty rows), one wave's five lanes per row: lane 5 g + r holds row r of the slice's g-th block.
+// The slice's blocks are stored as the wave reads them, 60 consecutive values per block column: the
+// diagonal and inverse blocks of slice s at 300 s + 60 j + lane, its off-diagonal blocks slot by slot
+// (its rows' k-th entries together, rows with fewer padded with zero blocks) at 300 slot + 60 j +
+// lane. The solve's vectors (the right-hand side, du, the GCR's directions) hold value q of position p
+// at 5 p + q, 60 values per slice; the padding rows' are 0.
 #pragma once
 
 #include "exact.hpp"
@@ -64,20 +67,14 @@ __device__ __forceinline__ void impl_cell_block(const double* __restrict__ dwdu,
   for (int q = 0; q < 25; ++q) b[q] = p[q];
 }
 
-// Five lanes per cell or face (12 per wave, lanes 60-63 idle), lane r computing row r of its blocks.
-constexpr int kRowGroups = kWave / 5;
+constexpr int kSlice = kWave / 5;          // rows per slice
+constexpr int kSliceVec = 5 * kSlice;      // values of a vector per slice, the lanes at work
+constexpr int kSliceBlock = 25 * kSlice;   // values of a slice's blocks
 
-__device__ __forceinline__ int impl_group_item(int& r) {
-  const int lane = threadIdx.x % kWave;
-  const int g = lane / 5;
-  r = lane % 5;
-  if (g >= kRowGroups) return -1;
-  return (blockIdx.x * (kBlock / kWave) + static_cast<int>(threadIdx.x / kWave)) * kRowGroups + g;
-}
-
-inline int impl_group_blocks(long long items) {
-  constexpr int per_block = (kBlock / kWave) * kRowGroups;
-  return static_cast<int>((items + per_block - 1) / per_block);
+// The address of value (0, 0) of entry e (its slot times kSlice plus its row's place in the slice);
+// value (r, j) is 60 j + r further.
+__device__ __forceinline__ long long impl_entry(int e) {
+  return static_cast<long long>(e / kSlice) * kSliceBlock + 5 * (e % kSlice);
 }
 
 // The diagonal blocks: lam_c / cfl on the diagonal, then the cell's faces in cell_faces order.
@@ -87,37 +84,42 @@ inline int impl_group_blocks(long long items) {
 // same sum from zero, negated exactly, and a running sum from +0 is never -0, so adding the
 // negated entry gives the bits of adding the product; it reads each entry's 25 contiguous values
 // instead of recomputing the product from the face blocks. A boundary face's term J_b D_c from
-// bj (25 x nb) and the cell's dW/dq block (cell-major). Five lanes per cell; stored at the cell's
-// row position.
+// bj (25 x nb) and the cell's dW/dq block (cell-major). One wave per slice, lane 5 g + r row r of the
+// g-th row's block; an empty row's block is 0.
 template <class C>
 __global__ __launch_bounds__(kBlock) void k_impl_diag(Dev<C> d, const double* __restrict__ dwdu,
                                                       const double* __restrict__ bj, const double* __restrict__ offd,
                                                       const int2* __restrict__ at, double cfl,
-                                                      const int* __restrict__ rank, double* __restrict__ diag) {
-  int r;
-  const int c = impl_group_item(r);
-  if (c < 0 || c >= d.nc) return;
+                                                      const int* __restrict__ cell, int slices,
+                                                      double* __restrict__ diag) {
+  const int lane = threadIdx.x % kWave;
+  const int s = blockIdx.x * (kBlock / kWave) + static_cast<int>(threadIdx.x / kWave);
+  if (s >= slices || lane >= kSliceVec) return;
+  const int r = lane % 5;
+  const int c = cell[kSlice * s + lane / 5];
   double dg[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  const double shift = static_cast<double>(d.lam[c]) / cfl;
-  dg[r] += shift;
-  for (int k = d.cfo[c]; k < d.cfo[c + 1]; ++k) {
-    const int e = d.inc[k];
-    const int f = e & 0x7fffffff;
-    if (f >= d.ni) {
-      double dc[25], j[5];
-      impl_cell_block(dwdu, c, dc);
-      impl_block_row(bj, d.nb, f - d.ni, 0, r, j);
-      impl_add_product_row(dg, j, dc, 1.0);
-    } else {
-      const int2 a = at[f];
-      const double* o = offd + 25LL * (e >= 0 ? a.y : a.x) + 5 * r;
+  if (c >= 0) {
+    const double shift = static_cast<double>(d.lam[c]) / cfl;
+    dg[r] += shift;
+    for (int k = d.cfo[c]; k < d.cfo[c + 1]; ++k) {
+      const int e = d.inc[k];
+      const int f = e & 0x7fffffff;
+      if (f >= d.ni) {
+        double dc[25], j[5];
+        impl_cell_block(dwdu, c, dc);
+        impl_block_row(bj, d.nb, f - d.ni, 0, r, j);
+        impl_add_product_row(dg, j, dc, 1.0);
+      } else {
+        const int2 a = at[f];
+        const double* o = offd + impl_entry(e >= 0 ? a.y : a.x) + r;
 #pragma unroll
-      for (int q = 0; q < 5; ++q) dg[q] += -o[q];
+        for (int q = 0; q < 5; ++q) dg[q] += -o[kSliceVec * q];
+      }
     }
   }
-  double* out = diag + 25LL * rank[c] + 5 * r;
+  double* out = diag + static_cast<long long>(kSliceBlock) * s + lane;
 #pragma unroll
-  for (int q = 0; q < 5; ++q) out[q] = dg[q];
+  for (int q = 0; q < 5; ++q) out[kSliceVec * q] = dg[q];
 }
 
 // The off-diagonal blocks of every interior face, at their entries (at[f].x in the owner's row,
@@ -139,18 +141,18 @@ __global__ __launch_bounds__(kBlock) void k_impl_off(Dev<C> d, const double* __r
   for (int q = 0; q < 25; ++q) out[q] = 0.0;
 #pragma unroll
   for (int r = 0; r < 5; ++r) impl_add_product_row(out + 5 * r, j + 5 * r, dm, 1.0);
-  double* up = offd + 25LL * k.x;
+  double* up = offd + impl_entry(k.x);
 #pragma unroll
-  for (int q = 0; q < 25; ++q) up[q] = out[q];
+  for (int q = 0; q < 25; ++q) up[kSliceVec * (q % 5) + q / 5] = out[q];
   impl_block(fj, d.ni, f, 0, j);
   impl_cell_block(dwdu, lr.x, dm);
 #pragma unroll
   for (int q = 0; q < 25; ++q) out[q] = 0.0;
 #pragma unroll
   for (int r = 0; r < 5; ++r) impl_add_product_row(out + 5 * r, j + 5 * r, dm, -1.0);
-  double* lo = offd + 25LL * k.y;
+  double* lo = offd + impl_entry(k.y);
 #pragma unroll
-  for (int q = 0; q < 25; ++q) lo[q] = out[q];
+  for (int q = 0; q < 25; ++q) lo[kSliceVec * (q % 5) + q / 5] = out[q];
 }
 
 // Each diagonal block's inverse: Gauss-Jordan on [A | I] with partial pivoting (the first row
@@ -162,13 +164,14 @@ __global__ __launch_bounds__(kBlock) void k_impl_invert(const double* __restrict
                                                         int* __restrict__ singular) {
   const int p = blockIdx.x * kBlock + threadIdx.x;
   if (p >= n) return;
-  const double* dp = diag + 25LL * p;
+  if (cell[p] < 0) return;  // an empty row: its inverse stays 0
+  const double* dp = diag + static_cast<long long>(kSliceBlock) * (p / kSlice) + 5 * (p % kSlice);
   double m[5][10];
 #pragma unroll
   for (int i = 0; i < 5; ++i) {
 #pragma unroll
     for (int j = 0; j < 5; ++j) {
-      m[i][j] = dp[5 * i + j];
+      m[i][j] = dp[kSliceVec * j + i];
       m[i][5 + j] = i == j ? 1.0 : 0.0;
     }
   }
@@ -212,109 +215,151 @@ __global__ __launch_bounds__(kBlock) void k_impl_invert(const double* __restrict
     }
   }
   if (!ok) atomicMin(singular, cell[p]);
-  double* ip = inverse + 25LL * p;
+  double* ip = inverse + static_cast<long long>(kSliceBlock) * (p / kSlice) + 5 * (p % kSlice);
 #pragma unroll
-  for (int i = 0; i < 5; ++i) {
+  for (int j = 0; j < 5; ++j) {
 #pragma unroll
-    for (int j = 0; j < 5; ++j) ip[5 * i + j] = m[i][5 + j];
+    for (int i = 0; i < 5; ++i) ip[kSliceVec * j + i] = m[i][5 + j];
   }
 }
 
-// The rows by position p (colour-major): cell[p] the row's cell, its entries off[p] .. off[p + 1]
-// (the cell's interior faces in ascending face order), entry k's block at offd + 25 k and its other
-// cell other[k].
+// The rows by position: the cell of each (-1: an empty row), slice s's slots slot[s] .. slot[s + 1],
+// and the position of the other cell of every entry (kSlice per slot; -1: padding). A row's entries
+// are the cell's interior faces in ascending face order, one per slot from the slice's first.
 struct ImplRows {
-  const int* off;    // n + 1
-  const int* other;  // 2 ni
-  const int* cell;   // n
+  const int* slot;
+  const int* other;
+  const int* cell;
 };
 
-// BlockMatrix::relax of one cell by a group of five lanes, lane q computing row q: x_c = D_c^-1
-// (b_c - sum_f A_cf x_other). Row q's sum runs over the faces, then j, in the one-thread order;
-// the group's five rows reach every lane of the group by shuffles for the inverse's product. Each
-// wave holds 12 groups (lanes 60-63 idle); every lane takes part in the shuffles.
-constexpr int kRelaxGroups = kWave / 5;
+// Sum over a slice's slots of A_cf x_other, row by row, added to (ADD) or taken from r: slot by slot,
+// then column by column, the one-thread order. kSlots slots' loads are issued together (the entry's
+// place, five block columns, one value of the other cell per lane; the group's five values reach its
+// lanes by shuffles), since the sums that use them are one chain. A padding entry is a zero block
+// times zeros, which leaves r's bits (a sum from +0, or r - 0) as they are.
+constexpr int kSlots = 6;
 
-__device__ __forceinline__ void impl_relax_rows(const ImplRows& rows, int p, bool active,
-                                                const double* __restrict__ offd, const double* __restrict__ inverse,
-                                                const double* __restrict__ b, double* __restrict__ x) {
-  const int lane = threadIdx.x % kWave;
-  const int q = lane % 5, base = lane - q;
-  const long long c = active ? rows.cell[p] : 0;
-  double r = 0.0;
-  if (active) {
-    r = b[5 * c + q];
-    for (int k = rows.off[p]; k < rows.off[p + 1]; ++k) {
-      const double* a = offd + 25LL * k + 5 * q;
-      const long long o = rows.other[k];
-      double xo[5];
+template <bool ADD>
+__device__ __forceinline__ double impl_slots(const ImplRows& rows, int s, int lane, const double* __restrict__ offd,
+                                             const double* x, double r) {
+  const bool on = lane < kSliceVec;
+  const int g = lane / 5, q = lane % 5, base = lane - q;
+  const int k1 = rows.slot[s + 1];
+  for (int k0 = rows.slot[s]; k0 < k1; k0 += kSlots) {
+    int o[kSlots];
+    double a[kSlots][5], xq[kSlots];
 #pragma unroll
-      for (int j = 0; j < 5; ++j) xo[j] = x[5 * o + j];
+    for (int u = 0; u < kSlots; ++u) {
+      const bool have = on && k0 + u < k1;
+      o[u] = have ? rows.other[kSlice * (k0 + u) + g] : -1;
 #pragma unroll
-      for (int j = 0; j < 5; ++j) r -= a[j] * xo[j];
+      for (int j = 0; j < 5; ++j) {
+        a[u][j] = have ? offd[static_cast<long long>(kSliceBlock) * (k0 + u) + kSliceVec * j + lane] : 0.0;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) xq[u] = o[u] >= 0 ? x[5LL * o[u] + q] : 0.0;
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) {
+      if (k0 + u >= k1) break;
+#pragma unroll
+      for (int j = 0; j < 5; ++j) {
+        const double xj = __shfl(xq[u], (base + j) % kWave);
+        if constexpr (ADD) {
+          r += a[u][j] * xj;
+        } else {
+          r -= a[u][j] * xj;
+        }
+      }
     }
   }
-  double rj[5];
-#pragma unroll
-  for (int j = 0; j < 5; ++j) rj[j] = __shfl(r, (base + j) % kWave);
-  if (active) {
-    const double* ip = inverse + 25LL * p + 5 * q;
-    double s = 0.0;
-#pragma unroll
-    for (int j = 0; j < 5; ++j) s += ip[j] * rj[j];
-    x[5 * c + q] = s;
-  }
+  return r;
 }
 
-// BlockMatrix::relax of the rows at positions first .. first + count (one colour): 12 cells per
-// wave.
+// BlockMatrix::relax of a slice's rows by one wave, lane 5 g + q row q of the g-th: x_c = D_c^-1 (b_c -
+// sum_f A_cf x_other). The group's five rows reach its lanes by shuffles for the inverse's product.
+// Bound by the blocks' bytes on a large colour and by the chain of loads (slot, place, value) on a
+// small one: the inverse, the right-hand side and six slots' blocks are in flight at once. With the
+// blocks row by row (each lane five consecutive values, a wave's loads 40 bytes apart) and one entry
+// in flight, two iterations of a 1.03M-cell channel took 54.1 ms where they now take 48.7 (the
+// relaxations 5.5 TB/s of blocks and values; two or three slots in flight 49.9 and 49.3 ms, each lane
+// reading the other cell's five values itself 54.2), a 39.5k-cell fp64 channel's 6.56 and 6.0 ms.
+__device__ __forceinline__ void impl_relax_slice(const ImplRows& rows, int s, const double* __restrict__ offd,
+                                                 const double* __restrict__ inverse, const double* __restrict__ b,
+                                                 double* x) {
+  const int lane = threadIdx.x % kWave;
+  const bool on = lane < kSliceVec;
+  const int base = lane - lane % 5;
+  const long long v = static_cast<long long>(kSliceVec) * s + lane;
+  double ip[5];
+#pragma unroll
+  for (int j = 0; j < 5; ++j) ip[j] = on ? inverse[static_cast<long long>(kSliceBlock) * s + kSliceVec * j + lane] : 0.0;
+  const double r = impl_slots<false>(rows, s, lane, offd, x, on ? b[v] : 0.0);
+  double sum = 0.0;
+#pragma unroll
+  for (int j = 0; j < 5; ++j) sum += ip[j] * __shfl(r, (base + j) % kWave);
+  if (on) x[v] = sum;
+}
+
+// The slice of this wave in a launch over `count` slices, -1 past them: each XCD takes a contiguous
+// run, whose neighbours' values share its L2.
+__device__ __forceinline__ int impl_slice(int count) {
+  const int waves = blockDim.x / kWave;
+  const int t = __builtin_amdgcn_readfirstlane(xcd_block() * waves + static_cast<int>(threadIdx.x / kWave));
+  return t < count ? t : -1;
+}
+
+// Threads of a block and blocks of a launch over `count` slices: four waves per block, or one where
+// that leaves fewer than two blocks per CU.
+constexpr int kImplFewSlices = 4 * 512;
+inline int impl_threads(int count) { return count < kImplFewSlices ? kWave : kBlock; }
+inline int impl_grid(int count) {
+  const int waves = impl_threads(count) / kWave;
+  return xcd_grid((count + waves - 1) / waves);
+}
+
+// BlockMatrix::relax of the slices first .. first + count (rows of one colour).
 __global__ __launch_bounds__(kBlock) void k_impl_relax(ImplRows rows, int first, int count,
                                                        const double* __restrict__ offd,
                                                        const double* __restrict__ inverse,
-                                                       const double* __restrict__ b, double* __restrict__ x) {
-  const int lane = threadIdx.x % kWave;
-  const int g = lane / 5;
-  const int t = (blockIdx.x * (kBlock / kWave) + static_cast<int>(threadIdx.x / kWave)) * kRelaxGroups + g;
-  const bool active = g < kRelaxGroups && t < count;
-  impl_relax_rows(rows, first + t, active, offd, inverse, b, x);
+                                                       const double* __restrict__ b, double* x) {
+  const int t = impl_slice(count);
+  if (t >= 0) impl_relax_slice(rows, first + t, offd, inverse, b, x);
 }
 
-// The first relaxation of the sweeps from x = 0, colour 0's `count` rows (positions 0 .. count):
-// x_c = D_c^-1 b_c, every neighbour's value being zero, without reading an off-diagonal block;
-// and x = 0 on the other rows up to n. The blocks are finite here (each is a term of a diagonal
-// block, and an inverse met a non-finite pivot otherwise and the solve was refused), so the products
-// left out are zeros; a zero's sign in b_c - 0 is lost in the inverse's product, whose sum starts at
-// +0.
-__global__ __launch_bounds__(kBlock) void k_impl_relax_start(ImplRows rows, int count, int n,
-                                                             const double* __restrict__ inverse,
+// The first relaxation of the sweeps from x = 0, colour 0's `count` slices: x_c = D_c^-1 b_c, every
+// neighbour's value being zero, without reading an off-diagonal block; and x = 0 on the other slices
+// up to n. The blocks are finite here (each is a term of a diagonal block, and an inverse met a
+// non-finite pivot otherwise and the solve was refused), so the products left out are zeros; a zero's
+// sign in b_c - 0 is lost in the inverse's product, whose sum starts at +0.
+__global__ __launch_bounds__(kBlock) void k_impl_relax_start(int count, int n, const double* __restrict__ inverse,
                                                              const double* __restrict__ b, double* __restrict__ x) {
-  int q;
-  const int p = impl_group_item(q);
-  if (p < 0 || p >= n) return;
-  const long long c = rows.cell[p];
-  double s = 0.0;
-  if (p < count) {
-    const double* ip = inverse + 25LL * p + 5 * q;
+  const int s = impl_slice(n);
+  if (s < 0) return;
+  const int lane = threadIdx.x % kWave;
+  const bool on = lane < kSliceVec;
+  const int base = lane - lane % 5;
+  const long long v = static_cast<long long>(kSliceVec) * s + lane;
+  double sum = 0.0;
+  if (s < count) {
+    const double r = on ? b[v] : 0.0;
 #pragma unroll
-    for (int j = 0; j < 5; ++j) s += ip[j] * b[5 * c + j];
+    for (int j = 0; j < 5; ++j) {
+      const double a = on ? inverse[static_cast<long long>(kSliceBlock) * s + kSliceVec * j + lane] : 0.0;
+      sum += a * __shfl(r, (base + j) % kWave);
+    }
   }
-  x[5 * c + q] = s;
+  if (on) x[v] = sum;
 }
 
-// Launch width of k_impl_relax for `count` cells.
-inline int impl_relax_blocks(int count) {
-  constexpr int per_block = (kBlock / kWave) * kRelaxGroups;
-  return (count + per_block - 1) / per_block;
-}
-
-// A run of small colours relaxed in order by one workgroup: phase p relaxes the rows at positions
-// first[p] .. first[p] + count[p], the barrier between phases making each phase's x visible to the next (the
+// A run of small colours relaxed in order by one workgroup: phase p relaxes the slices first[p] ..
+// first[p] + count[p], the barrier between phases making each phase's x visible to the next (the
 // workgroup shares one CU's cache), as separate launches would. Saves a launch per colour where a
 // colour is too small to fill the device.
 constexpr int kRelaxRunThreads = 1024;
 constexpr int kRelaxRunMax = 32;
-// Colours of at most this many cells (two passes of the run's workgroup) join a run.
-constexpr int kRelaxRunCells = 2 * (kRelaxRunThreads / kWave) * (kWave / 5);
+// Colours of at most this many slices (two passes of the run's workgroup) join a run.
+constexpr int kRelaxRunSlices = 2 * (kRelaxRunThreads / kWave);
 struct ImplRun {
   int first[kRelaxRunMax];
   int count[kRelaxRunMax];
@@ -324,44 +369,36 @@ struct ImplRun {
 __global__ __launch_bounds__(kRelaxRunThreads) void k_impl_relax_run(ImplRows rows, ImplRun run,
                                                                      const double* __restrict__ offd,
                                                                      const double* __restrict__ inverse,
-                                                                     const double* __restrict__ b,
-                                                                     double* __restrict__ x) {
-  constexpr int per_pass = (kRelaxRunThreads / kWave) * kRelaxGroups;
-  const int lane = threadIdx.x % kWave;
-  const int g = lane / 5;
-  const int slot = static_cast<int>(threadIdx.x / kWave) * kRelaxGroups + g;
+                                                                     const double* __restrict__ b, double* x) {
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
   for (int p = 0; p < run.phases; ++p) {
-    // wave-uniform trip count: every lane reaches the shuffles
-    for (int t0 = 0; t0 < run.count[p]; t0 += per_pass) {
-      const int t = t0 + slot;
-      const bool active = g < kRelaxGroups && t < run.count[p];
-      impl_relax_rows(rows, run.first[p] + t, active, offd, inverse, b, x);
+    for (int t = wave; t < run.count[p]; t += kRelaxRunThreads / kWave) {
+      impl_relax_slice(rows, run.first[p] + t, offd, inverse, b, x);
     }
     __syncthreads();
   }
 }
 
-// BlockMatrix::multiply: y_c = D_c x_c + sum_f A_cf x_other, the diagonal block first; five lanes
-// per row position (12 per wave), lane q summing row q in the one-thread order.
-__global__ __launch_bounds__(kBlock) void k_impl_multiply(ImplRows rows, int n, const double* __restrict__ diag,
+// BlockMatrix::multiply: y_c = D_c x_c + sum_f A_cf x_other, the diagonal block first, in slices as the
+// relaxation.
+__global__ __launch_bounds__(kBlock) void k_impl_multiply(ImplRows rows, int slices, const double* __restrict__ diag,
                                                           const double* __restrict__ offd,
                                                           const double* __restrict__ x, double* __restrict__ y) {
+  const int s = impl_slice(slices);
+  if (s < 0) return;
   const int lane = threadIdx.x % kWave;
-  const int g = lane / 5, q = lane % 5;
-  const int p = (blockIdx.x * (kBlock / kWave) + static_cast<int>(threadIdx.x / kWave)) * kRelaxGroups + g;
-  if (g >= kRelaxGroups || p >= n) return;
-  const long long c = rows.cell[p];
-  const double* dp = diag + 25LL * p + 5 * q;
+  const bool on = lane < kSliceVec;
+  const int base = lane - lane % 5;
+  const long long v = static_cast<long long>(kSliceVec) * s + lane;
+  const double xq = on ? x[v] : 0.0;
   double r = 0.0;
 #pragma unroll
-  for (int j = 0; j < 5; ++j) r += dp[j] * x[5 * c + j];
-  for (int k = rows.off[p]; k < rows.off[p + 1]; ++k) {
-    const double* a = offd + 25LL * k + 5 * q;
-    const long long o = rows.other[k];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) r += a[j] * x[5 * o + j];
+  for (int j = 0; j < 5; ++j) {
+    const double a = on ? diag[static_cast<long long>(kSliceBlock) * s + kSliceVec * j + lane] : 0.0;
+    r += a * __shfl(xq, (base + j) % kWave);
   }
-  y[5 * c + q] = r;
+  r = impl_slots<true>(rows, s, lane, offd, x, r);
+  if (on) y[v] = r;
 }
 
 // A block's exact-sum accumulator (carries resolved) added into the global words.
@@ -529,16 +566,18 @@ constexpr double kImplMinStep = 1e-6;
 // Each cell's admissible fraction (its density bound, then halved until its pressure bound holds),
 // and their least as the bits of a non-negative double (atomicMin of the bits).
 __global__ __launch_bounds__(kBlock) void k_impl_admissible(const double* __restrict__ u,
-                                                            const double* __restrict__ du, int n, double gamma,
+                                                            const double* __restrict__ du,
+                                                            const int* __restrict__ rank, int n, double gamma,
                                                             unsigned long long* __restrict__ bits) {
   const int c = blockIdx.x * kBlock + threadIdx.x;
   unsigned long long key = ~0ULL;
   if (c < n) {
+    const long long at = 5LL * rank[c];
     double v0[5], dv[5];
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       v0[k] = u[static_cast<long long>(k) * n + c];
-      dv[k] = du[5LL * c + k];
+      dv[k] = du[at + k];
     }
     double a = 1.0;
     if (dv[0] < 0.0) {
@@ -562,13 +601,13 @@ __global__ __launch_bounds__(kBlock) void k_impl_admissible(const double* __rest
 // sums, boundary values held), then over its boundary faces in cell_faces order, where the
 // reconstruction did not fall back to the cell value, bnd_jac applied to phi (grad_tan . r), and on
 // warped slip and wall faces the wall-warp term's tangent phi_p M^T grad_tan p.
-// dwdu cell-major (25 c + 5 i + j), v cell-major (5 c + j).
+// dwdu cell-major (25 c + 5 i + j), v by position (5 p + j).
 template <class C>
 __device__ __forceinline__ void impl_tangent(const double* __restrict__ dwdu, const double* __restrict__ v, long long c,
-                                             C* dw) {
+                                             long long p, C* dw) {
   C vc[5];
 #pragma unroll
-  for (int j = 0; j < 5; ++j) vc[j] = static_cast<C>(v[5 * c + j]);
+  for (int j = 0; j < 5; ++j) vc[j] = static_cast<C>(v[5 * p + j]);
 #pragma unroll
   for (int i = 0; i < 5; ++i) {
     C t = C(0);
@@ -582,11 +621,11 @@ __device__ __forceinline__ void impl_tangent(const double* __restrict__ dwdu, co
 // boundary term's stencils.
 template <class C>
 __global__ __launch_bounds__(kBlock) void k_impl_tangents(const double* __restrict__ dwdu, const double* __restrict__ v,
-                                                          int n, C* __restrict__ out) {
+                                                          const int* __restrict__ rank, int n, C* __restrict__ out) {
   const int c = blockIdx.x * kBlock + threadIdx.x;
   if (c >= n) return;
   C dw[5];
-  impl_tangent<C>(dwdu, v, c, dw);
+  impl_tangent<C>(dwdu, v, c, rank[c], dw);
 #pragma unroll
   for (int i = 0; i < 5; ++i) out[static_cast<long long>(i) * n + c] = dw[i];
 }
@@ -594,7 +633,7 @@ __global__ __launch_bounds__(kBlock) void k_impl_tangents(const double* __restri
 template <class C>
 __global__ __launch_bounds__(kBlock) void k_impl_bgrad(Dev<C> d, const int* __restrict__ cells, int count,
                                                        const C* __restrict__ tangents, const double* __restrict__ bj,
-                                                       double* __restrict__ y) {
+                                                       const int* __restrict__ rank, double* __restrict__ y) {
   const int t = blockIdx.x * kBlock + threadIdx.x;
   if (t >= count) return;
   const int c = cells[t];
@@ -668,16 +707,19 @@ __global__ __launch_bounds__(kBlock) void k_impl_bgrad(Dev<C> d, const int* __re
     }
   }
 #pragma unroll
-  for (int i = 0; i < 5; ++i) y[5 * static_cast<long long>(c) + i] += dres[i];
+  for (int i = 0; i < 5; ++i) y[5LL * rank[c] + i] += dres[i];
 }
 
 // ---- the GCR's vector operations (solvers/src/gcr.cpp), m values each
 
-// y = -x, x as the residual holds it (value q of cell c at q n + c), y cell-major (at 5 c + q).
-__global__ __launch_bounds__(kBlock) void k_impl_negate(const double* __restrict__ x, double* __restrict__ y,
-                                                        long long n) {
+// y = -x, x as the residual holds it (value q of cell c at q n + c), y by position (m values; an
+// empty row's are 0).
+__global__ __launch_bounds__(kBlock) void k_impl_negate(const double* __restrict__ x, const int* __restrict__ cell,
+                                                        double* __restrict__ y, long long n, long long m) {
   const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i < 5 * n) y[i] = -x[(i % 5) * n + i / 5];
+  if (i >= m) return;
+  const int c = cell[i / 5];
+  y[i] = c >= 0 ? -x[(i % 5) * n + c] : 0.0;
 }
 
 __global__ __launch_bounds__(kBlock) void k_impl_zero(double* __restrict__ x, long long m) {
@@ -700,11 +742,11 @@ __global__ void k_impl_scalar(const long long* __restrict__ words, const double*
   *out = den != nullptr ? v / *den : v;
 }
 
-// u += alpha du, u as the state holds it (value q of cell c at q n + c), du cell-major.
+// u += alpha du, u as the state holds it (value q of cell c at q n + c), du by position.
 __global__ __launch_bounds__(kBlock) void k_impl_update(double* __restrict__ u, const double* __restrict__ du,
-                                                        long long n, double alpha) {
+                                                        const int* __restrict__ rank, long long n, double alpha) {
   const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i < 5 * n) u[i] += alpha * du[5 * (i % n) + i / n];
+  if (i < 5 * n) u[i] += alpha * du[5LL * rank[i % n] + i / n];
 }
 
 }  // namespace mxe

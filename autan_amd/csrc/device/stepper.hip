@@ -342,7 +342,7 @@ class Stepper final : public StepperBase {
     have_jacobian_ = false;
     for (int q = 0; q < 5; ++q) report[q] = 0.0;
     const Dev<C> d = dev();
-    const long long m = 5LL * nc_;
+    const long long m = static_cast<long long>(kSliceVec) * slices_;
     const int gm = static_cast<int>((m + kBlock - 1) / kBlock);
     dot_next_ = 0;
     launch("impl_clear", [&] { k_impl_clear<<<1, 1024, 0, stream_>>>(words_.get(), kImplDots, bits_.get(), flag_.get()); });
@@ -352,14 +352,15 @@ class Stepper final : public StepperBase {
       });
     }
     launch("impl_diag", [&] {
-      k_impl_diag<C><<<impl_group_blocks(nc_), kBlock, 0, stream_>>>(d, jd_.get(), jb_.get(), offd_.get(), rat_.get(),
-                                                                     cfl, rank_.get(), diag_.get());
+      k_impl_diag<C><<<(slices_ + kBlock / kWave - 1) / (kBlock / kWave), kBlock, 0, stream_>>>(
+          d, jd_.get(), jb_.get(), offd_.get(), rat_.get(), cfl, ccells_.get(), slices_, diag_.get());
     });
     launch("impl_invert", [&] {
-      k_impl_invert<<<blocks(nc_), kBlock, 0, stream_>>>(diag_.get(), ccells_.get(), nc_, inv_.get(), flag_.get());
+      k_impl_invert<<<blocks(kSlice * static_cast<long long>(slices_)), kBlock, 0, stream_>>>(
+          diag_.get(), ccells_.get(), kSlice * slices_, inv_.get(), flag_.get());
     });
     launch("impl_zero", [&] { k_impl_zero<<<gm, kBlock, 0, stream_>>>(du_.get(), m); });
-    launch("impl_negate", [&] { k_impl_negate<<<gm, kBlock, 0, stream_>>>(res_.get(), kr_.get(), nc_); });
+    launch("impl_negate", [&] { k_impl_negate<<<gm, kBlock, 0, stream_>>>(res_.get(), ccells_.get(), kr_.get(), nc_, m); });
     int singular = INT32_MAX;
     check(hipMemcpyAsync(&singular, flag_.get(), sizeof(int), hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
     check(hipStreamSynchronize(stream_), "implicit_solve");
@@ -379,7 +380,7 @@ class Stepper final : public StepperBase {
       return;
     }
     launch("impl_admissible", [&] {
-      k_impl_admissible<<<blocks(nc_), kBlock, 0, stream_>>>(u_.get(), du_.get(), nc_, sc_.gamma, bits_.get());
+      k_impl_admissible<<<blocks(nc_), kBlock, 0, stream_>>>(u_.get(), du_.get(), rank_.get(), nc_, sc_.gamma, bits_.get());
     });
     unsigned long long abits = 0;
     check(hipMemcpyAsync(&abits, bits_.get(), sizeof(abits), hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
@@ -388,7 +389,7 @@ class Stepper final : public StepperBase {
     std::memcpy(&alpha, &abits, sizeof alpha);
     report[2] = alpha;
     if (alpha < kImplMinStep) return;
-    launch("impl_update", [&] { k_impl_update<<<gm, kBlock, 0, stream_>>>(u_.get(), du_.get(), nc_, alpha); });
+    launch("impl_update", [&] { k_impl_update<<<blocks(5LL * nc_), kBlock, 0, stream_>>>(u_.get(), du_.get(), rank_.get(), nc_, alpha); });
     prim_fresh_ = false;
     check(hipStreamSynchronize(stream_), "implicit_solve");
   }
@@ -398,19 +399,21 @@ class Stepper final : public StepperBase {
   int implicit_worst_cell() override {
     if (!implicit_ready_) throw std::invalid_argument("implicit_worst_cell: no implicit solve");
     const std::size_t n = static_cast<std::size_t>(nc_);
-    std::vector<double> u(5 * n), du(5 * n);
+    std::vector<double> u(5 * n), du(static_cast<std::size_t>(kSliceVec) * static_cast<std::size_t>(slices_));
+    std::vector<int> rank(n);
+    check(hipMemcpyAsync(rank.data(), rank_.get(), n * sizeof(int), hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
     u_.download(u.data(), u.size(), stream_);
     du_.download(du.data(), du.size(), stream_);
     check(hipStreamSynchronize(stream_), "implicit_worst_cell");
     auto pressure = [&](std::size_t c, double a) {
       double v[5];
-      for (std::size_t k = 0; k < 5; ++k) v[k] = u[k * n + c] + a * du[5 * c + k];  // du cell-major
+      for (std::size_t k = 0; k < 5; ++k) v[k] = u[k * n + c] + a * du[5 * std::size_t(rank[c]) + k];  // du by position
       return (sc_.gamma - 1.0) * (v[4] - 0.5 * (v[1] * v[1] + v[2] * v[2] + v[3] * v[3]) / v[0]);
     };
     std::size_t worst = 0;
     double lowest = std::numeric_limits<double>::infinity();
     for (std::size_t c = 0; c < n; ++c) {
-      const double r = std::min((u[c] + du[5 * c]) / u[c], pressure(c, 1.0) / pressure(c, 0.0));
+      const double r = std::min((u[c] + du[5 * std::size_t(rank[c])]) / u[c], pressure(c, 1.0) / pressure(c, 0.0));
       if (r < lowest) {
         lowest = r;
         worst = c;
@@ -468,12 +471,10 @@ class Stepper final : public StepperBase {
       colour_host_[c] = k;
       colours = std::max(colours, k + 1);
     }
-    std::vector<int> cells(std::max<std::size_t>(n, 1));
-    colour_off_.assign(static_cast<std::size_t>(colours) + 1, 0);
-    for (std::size_t c = 0; c < n; ++c) ++colour_off_[static_cast<std::size_t>(colour_host_[c]) + 1];
-    for (int k = 0; k < colours; ++k) colour_off_[static_cast<std::size_t>(k) + 1] += colour_off_[static_cast<std::size_t>(k)];
-    // Within a colour the cells with a neighbour of a higher colour come first (ascending), then the
-    // others: the way back down a sweep relaxes that prefix alone (plan_relax).
+    // The rows by position (implicit.hpp): colour by colour, in each the cells with a neighbour of a
+    // higher colour first (the way back down a sweep relaxes them alone, plan_relax), then the others;
+    // in each of these groups ascending, but within every 80 slices ordered by their entries, so that
+    // few slices pad rows of unlike lengths (2.6-9 % of the slots as they come, 0.2-0.7 % so).
     std::vector<char> above(n, 0);
     for (std::size_t c = 0; c < n; ++c) {
       for (int k = off[c]; k < off[c + 1]; ++k) {
@@ -481,16 +482,38 @@ class Stepper final : public StepperBase {
         if (colour_host_[static_cast<std::size_t>(other)] > colour_host_[c]) above[c] = 1;
       }
     }
-    std::vector<int> at(colour_off_.begin(), colour_off_.end() - 1);
-    colour_above_.assign(static_cast<std::size_t>(colours), 0);
-    for (const char first : {1, 0}) {
-      for (std::size_t c = 0; c < n; ++c) {
-        if (above[c] != first) continue;
-        const auto k = static_cast<std::size_t>(colour_host_[c]);
-        cells[static_cast<std::size_t>(at[k]++)] = static_cast<int>(c);
-        if (first) ++colour_above_[k];
+    std::vector<std::vector<int>> groups(2 * static_cast<std::size_t>(colours));
+    for (std::size_t c = 0; c < n; ++c) {
+      groups[2 * static_cast<std::size_t>(colour_host_[c]) + (above[c] ? 0 : 1)].push_back(static_cast<int>(c));
+    }
+    std::vector<int> cells, slot{0};
+    colour_off_.assign(1, 0);
+    colour_above_.clear();
+    auto entries = [&](int c) { return c < 0 ? 0 : off[static_cast<std::size_t>(c) + 1] - off[static_cast<std::size_t>(c)]; };
+    for (std::size_t g = 0; g < groups.size(); ++g) {
+      auto& rows = groups[g];
+      constexpr std::size_t kWindow = 80 * kSlice;
+      for (std::size_t w = 0; w < rows.size(); w += kWindow) {
+        std::stable_sort(rows.begin() + static_cast<std::ptrdiff_t>(w),
+                         rows.begin() + static_cast<std::ptrdiff_t>(std::min(rows.size(), w + kWindow)),
+                         [&](int a, int b) { return entries(a) < entries(b); });
+      }
+      rows.resize((rows.size() + kSlice - 1) / kSlice * kSlice, -1);
+      for (std::size_t p = 0; p < rows.size(); p += kSlice) {
+        int longest = 0;
+        for (std::size_t i = p; i < p + kSlice; ++i) longest = std::max(longest, entries(rows[i]));
+        slot.push_back(slot.back() + longest);
+      }
+      cells.insert(cells.end(), rows.begin(), rows.end());
+      const int end = static_cast<int>(cells.size() / kSlice);
+      if (g % 2 == 0) {
+        colour_above_.push_back(end - colour_off_.back());
+      } else {
+        colour_off_.push_back(end);
       }
     }
+    groups.clear();
+    slices_ = colour_off_.back();
     std::vector<int> bo;
     for (std::size_t c = 0; c < n; ++c) {
       for (int k = cfo_host_[c]; k < cfo_host_[c + 1]; ++k) {
@@ -502,39 +525,45 @@ class Stepper final : public StepperBase {
     }
     nbo_ = static_cast<int>(bo.size());
     if (nbo_ > 0) bocells_.upload(bo, stream_);
-    // The rows in the colour by colour order of `cells`: row p is cell cells[p]'s, its entries (the same
-    // ascending faces) numbered consecutively, so that a colour's rows and their blocks are one
-    // contiguous run; each interior face's two blocks sit at its entries in the two rows.
-    std::vector<int> rank(std::max<std::size_t>(n, 1)), poff(n + 1, 0);
-    for (std::size_t p = 0; p < n; ++p) {
-      const auto c = static_cast<std::size_t>(cells[p]);
-      rank[c] = static_cast<int>(p);
-      poff[p + 1] = poff[p] + (off[c + 1] - off[c]);
+    // Each interior face's entries in its two rows (slot times kSlice plus the row's place in its
+    // slice), a row's entries in ascending face order, and the other cell's position of each.
+    std::vector<int> rank(n);
+    for (std::size_t p = 0; p < cells.size(); ++p) {
+      if (cells[p] >= 0) rank[static_cast<std::size_t>(cells[p])] = static_cast<int>(p);
     }
-    std::vector<int> other(std::max<std::size_t>(2 * ni, 1));
+    const std::size_t slots = static_cast<std::size_t>(slot.back());
+    if (slots * kSlice > std::size_t(std::numeric_limits<int>::max())) throw std::invalid_argument("implicit step: too many faces");
+    std::vector<int> other(std::max<std::size_t>(slots * kSlice, 1), -1);
     std::vector<int2> face_at(std::max<std::size_t>(ni, 1));
-    std::vector<int> pfill(poff.begin(), poff.end() - 1);
+    std::vector<int> pfill(n, 0);
+    auto next_entry = [&](int c) {
+      const int p = rank[static_cast<std::size_t>(c)];
+      return kSlice * (slot[static_cast<std::size_t>(p / kSlice)] + pfill[static_cast<std::size_t>(c)]++) + p % kSlice;
+    };
     for (std::size_t f = 0; f < ni; ++f) {
       const int o = owner_host_[f], nb = neighbour_host_[f];
-      const int ko = pfill[static_cast<std::size_t>(rank[static_cast<std::size_t>(o)])]++;
-      const int kn = pfill[static_cast<std::size_t>(rank[static_cast<std::size_t>(nb)])]++;
-      other[static_cast<std::size_t>(ko)] = nb;
-      other[static_cast<std::size_t>(kn)] = o;
+      const int ko = next_entry(o), kn = next_entry(nb);
+      other[static_cast<std::size_t>(ko)] = rank[static_cast<std::size_t>(nb)];
+      other[static_cast<std::size_t>(kn)] = rank[static_cast<std::size_t>(o)];
       face_at[f] = make_int2(ko, kn);
     }
-    roff_.upload(poff, stream_);
+    rslot_.upload(slot, stream_);
     rother_.upload(other, stream_);
     rat_.upload(face_at, stream_);
     rank_.upload(rank, stream_);
     ccells_.upload(cells, stream_);
     plan_relax();
-    const std::size_t m = 5 * n;
+    const std::size_t m = static_cast<std::size_t>(kSliceVec) * static_cast<std::size_t>(slices_);
+    const std::size_t blk = static_cast<std::size_t>(kSliceBlock);
     jd_ = Buffer<double>(25 * n);
     jf_ = Buffer<double>(50 * std::max<std::size_t>(ni, 1));
     jb_ = Buffer<double>(25 * std::max<std::size_t>(static_cast<std::size_t>(nb_), 1));
-    diag_ = Buffer<double>(25 * n);
-    inv_ = Buffer<double>(25 * n);
-    offd_ = Buffer<double>(50 * std::max<std::size_t>(ni, 1));
+    diag_ = Buffer<double>(blk * static_cast<std::size_t>(slices_));
+    inv_ = Buffer<double>(blk * static_cast<std::size_t>(slices_));
+    offd_ = Buffer<double>(blk * std::max<std::size_t>(slots, 1));
+    // The padding's zeros, written once: no kernel writes there.
+    check(hipMemsetAsync(inv_.get(), 0, inv_.size() * sizeof(double), stream_), "hipMemsetAsync");
+    check(hipMemsetAsync(offd_.get(), 0, offd_.size() * sizeof(double), stream_), "hipMemsetAsync");
     kr_ = Buffer<double>(m);
     du_ = Buffer<double>(m);
     zs_ = Buffer<double>(m * kImplDirections);
@@ -543,7 +572,7 @@ class Stepper final : public StepperBase {
     bits_ = Buffer<unsigned long long>(2);
     flag_ = Buffer<int>(1);
     scalars_ = Buffer<double>(kImplScalars);
-    if (nbo_ > 0) tan_ = Buffer<C>(m);
+    if (nbo_ > 0) tan_ = Buffer<C>(5 * n);
     check(hipHostMalloc(reinterpret_cast<void**>(&host_scalars_), kImplScalars * sizeof(double), hipHostMallocDefault),
           "hipHostMalloc");
     check(hipStreamSynchronize(stream_), "implicit_setup");
@@ -555,13 +584,14 @@ class Stepper final : public StepperBase {
   void gauss_seidel(const double* b, double* z) {
     const ImplRows rows = impl_rows();
     launch("impl_relax_start", [&] {
-      k_impl_relax_start<<<impl_relax_blocks(nc_), kBlock, 0, stream_>>>(rows, colour_off_[1], nc_, inv_.get(), b, z);
+      k_impl_relax_start<<<impl_grid(slices_), impl_threads(slices_), 0, stream_>>>(colour_off_[1], slices_, inv_.get(),
+                                                                                    b, z);
     });
     for (const RelaxLaunch& l : relax_plan_) {
       if (l.run.phases == 0) {
         launch("impl_relax", [&] {
-          k_impl_relax<<<impl_relax_blocks(l.count), kBlock, 0, stream_>>>(rows, l.first, l.count, offd_.get(),
-                                                                           inv_.get(), b, z);
+          k_impl_relax<<<impl_grid(l.count), impl_threads(l.count), 0, stream_>>>(rows, l.first, l.count, offd_.get(),
+                                                                                  inv_.get(), b, z);
         });
       } else {
         launch("impl_relax_run", [&] {
@@ -571,7 +601,7 @@ class Stepper final : public StepperBase {
     }
   }
 
-  // The sweeps' colour sequence as launches: a colour of more than kRelaxRunCells cells is one
+  // The sweeps' colour sequence as launches: a colour of more than kRelaxRunSlices slices is one
   // launch over the device; consecutive smaller ones are one workgroup's run of phases.
   struct RelaxLaunch {
     int first = 0, count = 0;
@@ -594,7 +624,7 @@ class Stepper final : public StepperBase {
   // before, 54.1 ms with this plan (39.5k cells, fp64, second order: 7.23 and 6.56 ms).
   void plan_relax() {
     const int colours = static_cast<int>(colour_off_.size()) - 1;
-    std::vector<std::array<int, 2>> order;  // first position, rows
+    std::vector<std::array<int, 2>> order;  // first slice, slices
     for (int s = 0; s < kImplSweeps; ++s) {
       for (int k = 1; k < colours; ++k) {
         const int first = colour_off_[static_cast<std::size_t>(k)];
@@ -607,7 +637,7 @@ class Stepper final : public StepperBase {
     relax_plan_.clear();
     for (const auto& [first, count] : order) {
       if (count == 0) continue;
-      const bool small = count <= kRelaxRunCells;
+      const bool small = count <= kRelaxRunSlices;
       RelaxLaunch* last = relax_plan_.empty() ? nullptr : &relax_plan_.back();
       if (small && last != nullptr && last->run.phases > 0 && last->run.phases < kRelaxRunMax) {
         last->run.first[last->run.phases] = first;
@@ -665,17 +695,18 @@ class Stepper final : public StepperBase {
       gauss_seidel(kr_.get(), z);
       const ImplRows rows = impl_rows();
       launch("impl_multiply", [&] {
-        k_impl_multiply<<<impl_relax_blocks(nc_), kBlock, 0, stream_>>>(rows, nc_, diag_.get(), offd_.get(), z, w);
+        k_impl_multiply<<<impl_grid(slices_), impl_threads(slices_), 0, stream_>>>(rows, slices_, diag_.get(),
+                                                                                   offd_.get(), z, w);
       });
       // At second order the operator adds the boundary faces' gradient term.
       if (jac_second_ && nbo_ > 0) {
         const Dev<C> d = dev();
         launch("impl_tangents", [&] {
-          k_impl_tangents<C><<<blocks(nc_), kBlock, 0, stream_>>>(jd_.get(), z, nc_, tan_.get());
+          k_impl_tangents<C><<<blocks(nc_), kBlock, 0, stream_>>>(jd_.get(), z, rank_.get(), nc_, tan_.get());
         });
         launch("impl_bgrad", [&] {
           k_impl_bgrad<C><<<(nbo_ + kBlock - 1) / kBlock, kBlock, 0, stream_>>>(d, bocells_.get(), nbo_, tan_.get(),
-                                                                              jb_.get(), w);
+                                                                              jb_.get(), rank_.get(), w);
         });
       }
       // Modified Gram-Schmidt: beta_j = (w, w_j) / (w_j, w_j) on the w left by step j - 1, each
@@ -742,7 +773,7 @@ class Stepper final : public StepperBase {
     return std::isfinite(rr) ? std::sqrt(rr) / r0 : std::numeric_limits<double>::quiet_NaN();
   }
 
-  ImplRows impl_rows() const { return ImplRows{roff_.get(), rother_.get(), ccells_.get()}; }
+  ImplRows impl_rows() const { return ImplRows{rslot_.get(), rother_.get(), ccells_.get()}; }
 
   // A fresh exact-sum word set of the solve (cleared at its start).
   long long* next_words() {
@@ -755,7 +786,8 @@ class Stepper final : public StepperBase {
   Buffer<int> bocells_;
   int dot_next_ = 0;
   std::vector<int> colour_host_, colour_off_, colour_above_;
-  Buffer<int> roff_, rother_, rank_, ccells_, flag_;
+  int slices_ = 0;  // of the rows by position
+  Buffer<int> rslot_, rother_, rank_, ccells_, flag_;
   Buffer<int2> rat_;  // each interior face's two entries (owner's row, neighbour's row)
   Buffer<double> jd_, jf_, jb_, diag_, inv_, offd_, kr_, du_, zs_, ws_;
   Buffer<long long> words_;
