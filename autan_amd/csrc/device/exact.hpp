@@ -13,9 +13,9 @@
 // a result below 2^-1021 has fewer than 54 significant bits and was never rounded, and above it the
 // scaled value is normal.
 //
-// exact_value and its helpers are host and device functions when compiled as HIP: the device
-// rounds words it summed itself (the implicit solve's inner products) with the same code, so both
-// sides give the same double.
+// The rounding is a host and device function when compiled as HIP: the device rounds words it summed
+// itself (the implicit solve's inner products) with the same code, so both sides give the same
+// double.
 #pragma once
 
 #include <cmath>
@@ -35,21 +35,19 @@ inline constexpr int kExactLimbs = 68;
 inline constexpr int kExactWords = kExactLimbs + 3;
 inline constexpr int kExactBias = 1088;  // limb 0's weight is 2^-kExactBias
 
-// The value of exact words, rounded once to the nearest double (ties to even). Two passes over the
-// limbs in one register set (no digit array, so a device thread runs it without private memory):
-// the first resolves the carries only to learn the sign; the second resolves them again into the
-// base-2^32 digits of |sum| (two's complement on the fly when negative) and keeps the highest
-// non-zero digit, the two digits under it and whether any digit below those is non-zero.
-MXE_HOST_DEVICE inline double exact_value(const long long* in) {
+// The value of limbs [first, last) (`limb(i)`; the others zero, at least one of these not), rounded
+// once to the nearest double (ties to even). Two passes over them in one register set (no digit
+// array, so a device thread runs it without private memory): the first resolves the carries only to
+// learn the sign; the second resolves them again into the base-2^32 digits of |sum| (two's complement
+// on the fly when negative) and keeps the highest non-zero digit, the two digits under it and whether
+// any digit below those is non-zero. Both go three limbs past `last` (or to the end), where a carry
+// below 2^32 in magnitude has become 0 or -1 and the complement's +1 has been taken.
+template <class Limb>
+MXE_HOST_DEVICE inline double exact_round(const Limb& limb, int first, int last) {
   constexpr double inf = std::numeric_limits<double>::infinity();
-  const long long pos_inf = in[kExactLimbs], neg_inf = in[kExactLimbs + 1], nans = in[kExactLimbs + 2];
-  if (nans > 0 || (pos_inf > 0 && neg_inf > 0)) return std::numeric_limits<double>::quiet_NaN();
-  if (pos_inf > 0) return inf;
-  if (neg_inf > 0) return -inf;
-  // Unrolled: the limbs' loads do not wait on the carry chain.
+  const int end = last + 3 < kExactLimbs ? last + 3 : kExactLimbs;
   __int128 carry = 0;
-#pragma GCC unroll 68
-  for (int i = 0; i < kExactLimbs; ++i) carry = (carry + in[i]) >> 32;  // floor division
+  for (int i = first; i < end; ++i) carry = (carry + limb(i)) >> 32;  // floor division
   const bool negative = carry < 0;
   carry = 0;
   unsigned long long up = 1;  // the +1 of the two's complement, carried up the digits
@@ -58,9 +56,8 @@ MXE_HOST_DEVICE inline double exact_value(const long long* in) {
   int top_index = -1;                              // the highest non-zero digit so far
   std::uint32_t top0 = 0, top1 = 0, top2 = 0;      // that digit and the two under it
   bool top_sticky = false;                         // any non-zero digit under those three
-#pragma GCC unroll 68
-  for (int i = 0; i < kExactLimbs; ++i) {
-    const __int128 acc = carry + in[i];
+  for (int i = first; i < end; ++i) {
+    const __int128 acc = carry + limb(i);
     std::uint32_t digit = static_cast<std::uint32_t>(static_cast<unsigned __int128>(acc) & 0xffffffffu);
     carry = acc >> 32;
     if (negative) {
@@ -101,6 +98,59 @@ MXE_HOST_DEVICE inline double exact_value(const long long* in) {
   const double magnitude = std::ldexp(rounded, lead - 63 - kExactBias);
   return negative ? -magnitude : magnitude;
 }
+
+// A sum's value by its counts of +inf, -inf and NaN terms; false where they do not decide it.
+MXE_HOST_DEVICE inline bool exact_special(long long pos_inf, long long neg_inf, long long nans, double& value) {
+  constexpr double inf = std::numeric_limits<double>::infinity();
+  if (nans > 0 || (pos_inf > 0 && neg_inf > 0)) {
+    value = std::numeric_limits<double>::quiet_NaN();
+  } else if (pos_inf > 0) {
+    value = inf;
+  } else if (neg_inf > 0) {
+    value = -inf;
+  } else {
+    return false;
+  }
+  return true;
+}
+
+// The value of exact words.
+inline double exact_value(const long long* in) {
+  double value = 0.0;
+  if (exact_special(in[kExactLimbs], in[kExactLimbs + 1], in[kExactLimbs + 2], value)) return value;
+  int first = 0, last = kExactLimbs;
+  while (first < last && in[first] == 0) ++first;
+  while (last > first && in[last - 1] == 0) --last;
+  if (first == last) return 0.0;
+  return exact_round([in](int i) { return in[i]; }, first, last);
+}
+
+#if defined(__HIP__)
+// exact_value by one whole wave (every lane active and given the same words; every lane returns the
+// value): the lanes hold the limbs, find the non-zero ones together, and the rounding's chain runs
+// over those few with each limb read from its lane. A product sum of a solve fills 4 to 8 limbs; over
+// all 68, one thread took 10 us of every kernel that begins by rounding a sum.
+__device__ inline double exact_value_wave(const long long* __restrict__ in) {
+  const int lane = static_cast<int>(threadIdx.x) % 64;
+  const long long a = in[lane];
+  const long long b = 64 + lane < kExactWords ? in[64 + lane] : 0;
+  auto at = [&](int i) {
+    const long long v = i < 64 ? a : b;
+    const int lo = __builtin_amdgcn_readlane(static_cast<int>(v), i % 64);
+    const int hi = __builtin_amdgcn_readlane(static_cast<int>(v >> 32), i % 64);
+    return static_cast<long long>((static_cast<unsigned long long>(static_cast<unsigned int>(hi)) << 32) |
+                                  static_cast<unsigned int>(lo));
+  };
+  double value = 0.0;
+  if (exact_special(at(kExactLimbs), at(kExactLimbs + 1), at(kExactLimbs + 2), value)) return value;
+  const unsigned long long low = __ballot(a != 0);
+  const unsigned long long high = __ballot(64 + lane < kExactLimbs && b != 0);
+  if (low == 0 && high == 0) return 0.0;
+  const int first = low != 0 ? __ffsll(low) - 1 : 64 + __ffsll(high) - 1;
+  const int last = high != 0 ? 64 + 64 - __clzll(high) : 64 - __clzll(low);
+  return exact_round(at, first, last);
+}
+#endif
 
 // A running exact sum on the host, in the same words.
 class ExactSum {

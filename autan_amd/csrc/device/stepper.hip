@@ -248,7 +248,7 @@ class Stepper final : public StepperBase {
     (void)hipStreamSynchronize(stream_);
     drop_graphs();
     if (host_small_ != nullptr) (void)hipHostFree(host_small_);
-    if (host_scalars_ != nullptr) (void)hipHostFree(host_scalars_);
+    if (host_words_ != nullptr) (void)hipHostFree(host_words_);
     if (ev_in_ != nullptr) (void)hipEventDestroy(ev_in_);
     if (ev_out_ != nullptr) (void)hipEventDestroy(ev_out_);
     if (own_stream_) (void)hipStreamDestroy(stream_);
@@ -345,7 +345,8 @@ class Stepper final : public StepperBase {
     const long long m = static_cast<long long>(kSliceVec) * slices_;
     const int gm = static_cast<int>((m + kBlock - 1) / kBlock);
     dot_next_ = 0;
-    launch("impl_clear", [&] { k_impl_clear<<<1, 1024, 0, stream_>>>(words_.get(), kImplDots, bits_.get(), flag_.get()); });
+    launch("impl_clear", [&] { k_impl_clear<<<1, 1024, 0, stream_>>>(words_.get(), static_cast<int>(words_.size()), bits_.get(), flag_.get());
+    });
     if (ni_ > 0) {
       launch("impl_off", [&] {
         k_impl_off<C><<<blocks(ni_), kBlock, 0, stream_>>>(d, jd_.get(), jf_.get(), rat_.get(), offd_.get());
@@ -433,9 +434,11 @@ class Stepper final : public StepperBase {
   static constexpr int kImplDirections = 10;
   static constexpr double kImplTolerance = 0.1;
   static constexpr double kImplFailure = 0.9;
-  // The exact inner products one solve can take: the first, then per direction k its k
-  // orthogonalisation coefficients, its norm, its step and the new residual's norm.
-  static constexpr int kImplDots = 1 + kImplDirections * (kImplDirections - 1) / 2 + 3 * kImplDirections;
+  // The exact inner products one solve can take whose words stay on the device: per direction k its k
+  // orthogonalisation coefficients, its norm and its step. After them the words the host reads: the
+  // first residual's (r, r), then per direction (w, w) rounded and the new residual's (r, r).
+  static constexpr int kImplDots = kImplDirections * (kImplDirections - 1) / 2 + 2 * kImplDirections;
+  static constexpr int kImplHostWords = kWords + kImplDirections * (1 + kWords);
 
   // Buffers, the rows (each cell's interior faces in ascending face order: BlockMatrix's lists) and
   // the greedy colouring in cell order, made on the first implicit call.
@@ -568,12 +571,11 @@ class Stepper final : public StepperBase {
     du_ = Buffer<double>(m);
     zs_ = Buffer<double>(m * kImplDirections);
     ws_ = Buffer<double>(m * kImplDirections);
-    words_ = Buffer<long long>(std::size_t(kImplDots) * kWords);
+    words_ = Buffer<long long>(std::size_t(kImplDots) * kWords + kImplHostWords);
     bits_ = Buffer<unsigned long long>(2);
     flag_ = Buffer<int>(1);
-    scalars_ = Buffer<double>(kImplScalars);
     if (nbo_ > 0) tan_ = Buffer<C>(5 * n);
-    check(hipHostMalloc(reinterpret_cast<void**>(&host_scalars_), kImplScalars * sizeof(double), hipHostMallocDefault),
+    check(hipHostMalloc(reinterpret_cast<void**>(&host_words_), kImplHostWords * sizeof(long long), hipHostMallocDefault),
           "hipHostMalloc");
     check(hipStreamSynchronize(stream_), "implicit_setup");
     implicit_ready_ = true;
@@ -662,16 +664,18 @@ class Stepper final : public StepperBase {
   }
 
   // Gcr::solve (solvers/src/gcr.cpp) on kr_ = -R into du_ = 0: returns the residual drop. The
-  // scalars (inner products rounded by exact_value, the Gram-Schmidt and step coefficients) are
-  // computed and used on the device, each inner product fused into the vector update before it
-  // (exact sums: the same bits in any order); the host reads (w, w) and (r, r) once per direction
-  // for the stopping rules, and takes every decision the host loop takes, on the same values.
+  // Gram-Schmidt and step coefficients are rounded and used on the device, each inner product fused
+  // into the vector update before it (exact sums: the same bits in any order); the host reads (w, w)
+  // and the words of (r, r) once per direction for the stopping rules, and takes every decision the
+  // host loop takes, on the same values.
   double gcr(long long m, int gm, int& cycles) {
-    double* sc = scalars_.get();  // [0, D) (w_k, w_k), then alpha, (r, r), (r_0, r_0)
-    constexpr int kAlpha = kImplDirections, kRr = kAlpha + 1, kR0 = kRr + 1;
-    static_assert(kR0 + 1 == kImplScalars);
-    // Grid of the kernels with exact sums: about 8 values per thread (each block resolves its
-    // limbs' carries serially before adding them), at most 1024 blocks.
+    // What the host reads of direction k: (w_k, w_k), which the next directions divide by, and the
+    // words of (r, r), which the host rounds; direction 0's stand after the words of (r_0, r_0).
+    auto ww_at = [](int k) { return kWords + k * (1 + kWords); };
+    long long* hw = words_.get() + std::size_t(kImplDots) * kWords;
+    auto ww_of = [&](int k) { return reinterpret_cast<double*>(hw + ww_at(k)); };
+    // Grid of the kernels with exact sums: about 8 values per thread (a block's words cost it a
+    // fixed time), at most 1024 blocks.
     const int gd = static_cast<int>(std::max<long long>(1, std::min<long long>(1024, m / (8LL * kBlock))));
     unsigned long long mbits = 0;
     launch("impl_maxabs", [&] { k_impl_maxabs<<<gd, kBlock, 0, stream_>>>(kr_.get(), m, bits_.get() + 1); });
@@ -684,9 +688,7 @@ class Stepper final : public StepperBase {
     if (scale == 0.0) return 0.0;
     launch("impl_scale", [&] { k_impl_scale<<<gm, kBlock, 0, stream_>>>(kr_.get(), m, scale, 0); });
     {
-      long long* w0 = next_words();
-      launch("impl_dot", [&] { k_impl_dot<<<gd, kBlock, 0, stream_>>>(kr_.get(), kr_.get(), m, w0); });
-      launch("impl_scalar", [&] { k_impl_scalar<<<1, kWave, 0, stream_>>>(w0, nullptr, sc + kR0); });
+      launch("impl_dot", [&] { k_impl_dot<<<gd, kBlock, 0, stream_>>>(kr_.get(), kr_.get(), m, hw); });
     }
     double r0 = 0.0, rr = 0.0;
     for (int k = 0; k < kImplDirections; ++k) {
@@ -715,59 +717,56 @@ class Stepper final : public StepperBase {
       long long* prev = nullptr;
       long long* ww_words = nullptr;
       long long* rw_words = nullptr;
-      if (k == 0) {
+      auto orth_last = [&](const double* zj, const double* wj, const double* den) {
         ww_words = next_words();
         rw_words = next_words();
         launch("impl_orth_dots", [&] {
-          k_impl_orth_dots<<<gd, kBlock, 0, stream_>>>(z, w, nullptr, nullptr, m, nullptr, nullptr, w, ww_words,
-                                                      kr_.get(), rw_words);
+          k_impl_orth_dots<2><<<gd, kBlock, 0, stream_>>>(z, w, zj, wj, m, prev, den, w, ww_words, kr_.get(), rw_words);
         });
-      } else {
-        prev = next_words();
+      };
+      auto orth_next = [&](const double* zj, const double* wj, const double* den, int j) {
+        long long* nxt = next_words();
+        const double* wn = ws_.get() + std::size_t(j) * std::size_t(m);
         launch("impl_orth_dots", [&] {
-          k_impl_orth_dots<<<gd, kBlock, 0, stream_>>>(z, w, nullptr, nullptr, m, nullptr, nullptr, ws_.get(), prev,
-                                                      nullptr, nullptr);
+          k_impl_orth_dots<1><<<gd, kBlock, 0, stream_>>>(z, w, zj, wj, m, prev, den, wn, nxt, nullptr, nullptr);
         });
+        prev = nxt;
+      };
+      if (k == 0) {
+        orth_last(nullptr, nullptr, nullptr);
+      } else {
+        orth_next(nullptr, nullptr, nullptr, 0);
       }
       for (int j = 0; j < k; ++j) {
         const double* zj = zs_.get() + std::size_t(j) * std::size_t(m);
         const double* wj = ws_.get() + std::size_t(j) * std::size_t(m);
         if (j + 1 < k) {
-          long long* nxt = next_words();
-          const double* wn = ws_.get() + std::size_t(j + 1) * std::size_t(m);
-          launch("impl_orth_dots", [&] {
-            k_impl_orth_dots<<<gd, kBlock, 0, stream_>>>(z, w, zj, wj, m, prev, sc + j, wn, nxt, nullptr, nullptr);
-          });
-          prev = nxt;
+          orth_next(zj, wj, ww_of(j), j + 1);
         } else {
-          ww_words = next_words();
-          rw_words = next_words();
-          launch("impl_orth_dots", [&] {
-            k_impl_orth_dots<<<gd, kBlock, 0, stream_>>>(z, w, zj, wj, m, prev, sc + j, w, ww_words, kr_.get(),
-                                                        rw_words);
-          });
+          orth_last(zj, wj, ww_of(j));
         }
       }
-      long long* rr_words = next_words();
       launch("impl_advance_dot", [&] {
         k_impl_advance_dot<<<gd, kBlock, 0, stream_>>>(du_.get(), kr_.get(), z, w, m, bits_.get() + 1, ww_words,
-                                                      rw_words, sc + k, sc + kAlpha, rr_words);
+                                                      rw_words, ww_of(k), hw + ww_at(k) + 1);
       });
-      launch("impl_scalar", [&] { k_impl_scalar<<<1, kWave, 0, stream_>>>(rr_words, nullptr, sc + kRr); });
-      check(hipMemcpyAsync(host_scalars_, sc, (kR0 + 1) * sizeof(double), hipMemcpyDeviceToHost, stream_),
+      const int from = k == 0 ? 0 : ww_at(k), to = ww_at(k + 1);
+      check(hipMemcpyAsync(host_words_ + from, hw + from, std::size_t(to - from) * sizeof(long long),
+                           hipMemcpyDeviceToHost, stream_),
             "hipMemcpyAsync");
       check(hipStreamSynchronize(stream_), "implicit_solve");
       if (k == 0) {
-        r0 = std::sqrt(host_scalars_[kR0]);
+        r0 = std::sqrt(exact_value(host_words_));
         rr = r0 * r0;
       }
-      const double ww = host_scalars_[k];
+      double ww;
+      std::memcpy(&ww, host_words_ + ww_at(k), sizeof ww);
       cycles = k + 1;
       if (!(ww > 0.0)) {
         if (!std::isfinite(ww)) rr = ww;
         break;
       }
-      rr = host_scalars_[kRr];
+      rr = exact_value(host_words_ + ww_at(k) + 1);
       if (std::sqrt(rr) <= kImplTolerance * r0) break;
     }
     return std::isfinite(rr) ? std::sqrt(rr) / r0 : std::numeric_limits<double>::quiet_NaN();
@@ -792,10 +791,7 @@ class Stepper final : public StepperBase {
   Buffer<double> jd_, jf_, jb_, diag_, inv_, offd_, kr_, du_, zs_, ws_;
   Buffer<long long> words_;
   Buffer<unsigned long long> bits_;
-  // The GCR's scalars on the device and the pinned host copy of the ones the host reads.
-  static constexpr int kImplScalars = kImplDirections + 3;
-  Buffer<double> scalars_;
-  double* host_scalars_ = nullptr;
+  long long* host_words_ = nullptr;  // the pinned copy of the words and scalars the host reads
   Buffer<C> tan_;  // the boundary term's primitive tangents
 
  public:
