@@ -15,6 +15,7 @@
 #include <random>
 #include <stdexcept>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "../../../include/mxmlp.h"
@@ -238,28 +239,57 @@ __global__ void k_fill(float* __restrict__ p, long long n, float v) {
   if (i < n) p[i] = v;
 }
 
-// Adam (Kingma and Ba 2015) on the FP32 master weights, then their BF16 copy. `mask` marks the
-// entries that exist (padding stays zero); the bias corrections are the step state's.
-__global__ void k_adam(float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m1, float* __restrict__ m2,
-                       const unsigned char* __restrict__ mask, long long n, float lr, float b1, float b2, float eps,
-                       const StepState* __restrict__ st, bf16* __restrict__ wb) {
-  const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n) return;
+// The splits' partial gradients added in split order.
+__device__ __forceinline__ float sum_parts(const float* __restrict__ part, long long np, int splits, long long i) {
+  float v = 0.0f;
+#pragma unroll 8
+  for (int q = 0; q < splits; ++q) v += part[q * np + i];
+  return v;
+}
+
+// The BF16 weights three times over: row-major for the layer-by-layer products, and as the operands of
+// the fused kernels, packed (pack_place) as they are and transposed, at the places `at` gives each
+// parameter (x the packed copy's, y the transposed one's, -1: none).
+struct WeightCopies {
+  bf16* row;
+  bf16* packed;
+  bf16* turned;
+  const int2* at;
+};
+
+__device__ __forceinline__ void store_copies(const WeightCopies& c, long long i, float w) {
+  const bf16 v = static_cast<bf16>(w);
+  const int2 p = c.at[i];
+  c.row[i] = v;
+  if (p.x >= 0) c.packed[p.x] = v;
+  if (p.y >= 0) c.turned[p.y] = v;
+}
+
+// Adam (Kingma and Ba 2015) on the FP32 master weights, then their BF16 copies. `mask` marks the entries that exist (padding stays zero); the
+// bias corrections are the step state's. The gradient is the sum of `splits` partial ones, in the order
+// `order` gives (place j is parameter order[j]; null: the parameters').
+__global__ void k_adam(float* __restrict__ w, const float* __restrict__ part, int splits,
+                       const int* __restrict__ order, float* __restrict__ m1,
+                       float* __restrict__ m2, const unsigned char* __restrict__ mask, long long n, float lr, float b1,
+                       float b2, float eps, const StepState* __restrict__ st, WeightCopies copies) {
+  const long long j = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (j >= n) return;
+  const long long i = order != nullptr ? order[j] : j;
   const float c1 = st->c1, c2 = st->c2;
   if (mask[i]) {
-    const float gi = g[i];
+    const float gi = sum_parts(part, n, splits, j);
     const float a = b1 * m1[i] + (1.0f - b1) * gi;
     const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
     m1[i] = a;
     m2[i] = b;
     w[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
   }
-  if (wb != nullptr) wb[i] = static_cast<bf16>(w[i]);
+  store_copies(copies, i, w[i]);
 }
 
-__global__ void k_to_bf16(const float* __restrict__ w, long long n, bf16* __restrict__ wb) {
+__global__ void k_to_bf16(const float* __restrict__ w, long long n, WeightCopies copies) {
   const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) wb[i] = static_cast<bf16>(w[i]);
+  if (i < n) store_copies(copies, i, w[i]);
 }
 
 // Network outputs back in physical units: y * scale + mean for the first d columns.
@@ -270,6 +300,18 @@ __global__ void k_out(const float* __restrict__ y, int n, int d, int width, cons
   const long long r = i / d;
   const int c = static_cast<int>(i % d);
   out[i] = y[r * width + c] * scale[c] + mean[c];
+}
+
+// The fused kernels' weights: for each 16 outputs and each 32 inputs (of `steps` such) the 1 KB that a
+// wave reads as one matrix-core operand, lane l the eight inputs 8 (l / 16) .. of output l mod 16. A
+// load is then eight consecutive cache lines, in eight of the L2's channels; read from rows of 512
+// bytes, sixteen half lines in four channels, every CU's loads of a layer queued on those.
+__host__ __device__ constexpr long long pack_place(int out, int in, int steps) {
+  return ((static_cast<long long>(out / 16) * steps + in / 32) * 64 + in % 32 / 8 * 16 + out % 16) * 8 + in % 8;
+}
+// The operand of outputs 16 tile .. and inputs 32 step .. for this lane.
+__device__ __forceinline__ bf16x8 packed_operand(const bf16* W, int tile, int step, int steps) {
+  return *reinterpret_cast<const bf16x8*>(W + ((static_cast<long long>(tile) * steps + step) * 64 + threadIdx.x % 64) * 8);
 }
 
 // The layers of a network as k_infer reads them: weight and bias offsets into the parameter arrays.
@@ -318,21 +360,18 @@ __global__ __launch_bounds__(64 * WAVES) void k_infer(const float* __restrict__ 
 #pragma unroll
         for (int j = 0; j < CT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
-      const int nb = wave * 16 * CT;
-      const bf16* wrow[CT];
-#pragma unroll
-      for (int j = 0; j < CT; ++j) wrow[j] = W + static_cast<long long>(nb + 16 * j + row) * K + kq;
+      const int nb = wave * 16 * CT, steps = K / kTileK;
       // The next K step's weights are in flight while this step's products run.
       bf16x8 b_next[CT];
 #pragma unroll
-      for (int j = 0; j < CT; ++j) b_next[j] = *reinterpret_cast<const bf16x8*>(wrow[j]);
+      for (int j = 0; j < CT; ++j) b_next[j] = packed_operand(W, wave * CT + j, 0, steps);
       for (int k0 = 0; k0 < K; k0 += kTileK) {
         bf16x8 b[CT];
 #pragma unroll
         for (int j = 0; j < CT; ++j) b[j] = b_next[j];
         if (k0 + kTileK < K) {
 #pragma unroll
-          for (int j = 0; j < CT; ++j) b_next[j] = *reinterpret_cast<const bf16x8*>(wrow[j] + k0 + kTileK);
+          for (int j = 0; j < CT; ++j) b_next[j] = packed_operand(W, wave * CT + j, k0 / kTileK + 1, steps);
         }
 #pragma unroll
         for (int i = 0; i < RT; ++i) {
@@ -366,7 +405,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_infer(const float* __restrict__ 
         f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
         for (int k0 = 0; k0 < K; k0 += kTileK) {
           const bf16x8 a = *reinterpret_cast<const bf16x8*>(&act[(16 * i + row) * ld + k0 + kq]);
-          const bf16x8 b = *reinterpret_cast<const bf16x8*>(W + static_cast<long long>(row) * K + k0 + kq);
+          const bf16x8 b = packed_operand(W, 0, k0 / kTileK, K / kTileK);
           acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc, 0, 0, 0);
         }
         const int nn = lane % 16;
@@ -417,6 +456,369 @@ void launch_infer_rows(int rows, const float* x, int n, int d_in, int d_out, con
       break;
     default: throw std::invalid_argument("inference tile: 64, 96 or 128 samples per workgroup");
   }
+}
+
+// ------------------------------------------------------------------------ the fused training step
+//
+// One batch is three kernels (hidden widths up to 256): k_train, the forward, the loss and the
+// backward's dZ chain of 32 samples per workgroup, the samples' activations and gradients in LDS; k_dw,
+// every layer's weight and bias gradients; k_adam, which adds k_dw's partial sums and takes Adam's
+// step. What k_dw contracts over the samples, the activations H and the gradients dZ, is stored by
+// k_train as k_dw's matrix-core operands read it: for each tile of 32 samples and each feature four
+// packs of eight samples, pack g the samples 4 g .. + 3 and 16 + 4 g .. + 3 (what one lane of a 16 x 16
+// product over two row tiles holds of a feature), so that k_dw needs no transposition and no LDS.
+constexpr int kPackTile = 32;
+
+// The training step's places: `hidden` layers of width H after 32 inputs, 16 outputs (padded widths),
+// `rows` samples (whole tiles). Worked out rather than read from a table in the kernel's arguments,
+// whose first reads a workgroup waits on one after the other.
+struct TrainPlan {
+  int hidden, width;
+  long long rows;
+  // Layer l's weights in the parameters (its biases follow them), l = 0 .. hidden.
+  __host__ __device__ long long w(int l) const {
+    const long long H = width;
+    return l == 0 ? 0 : 33 * H + (l - 1) * (H * H + H);
+  }
+  __host__ __device__ long long b(int l) const {
+    return w(l) + static_cast<long long>(l == 0 ? 32 : width) * (l == hidden ? 16 : width);
+  }
+  // The transposed weights of layer l = 1 .. hidden (outputs and inputs exchanged; the output layer's
+  // 16 outputs filled up to 32 with zeros).
+  __host__ __device__ long long wt(int l) const { return static_cast<long long>(l - 1) * width * width; }
+  // Where the partial gradients hold the weight of layer l from input k into output n: 16 x 16 products,
+  // lane 16 (n mod 16 / 4) + k mod 16 of each four consecutive outputs. Biases stand at b(l) + n.
+  long long part_place(int l, int n, int k) const {
+    const int kf = (l == 0 ? 32 : width) / 16;
+    return w(l) + ((static_cast<long long>(n / 16) * kf + k / 16) * 64 + n % 16 / 4 * 16 + k % 16) * 4 + n % 4;
+  }
+  // The packs of H_l and dZ_l.
+  __host__ __device__ long long h(int l) const { return rows * (l == 0 ? 0 : 32 + width + (l - 1) * 2LL * width); }
+  __host__ __device__ long long dz(int l) const { return h(l) + rows * (l == 0 ? 32 : width); }
+};
+
+// Where a traced batch's tensors go, row-major by layer (for tests): inputs, pre-activations, dZ.
+struct TraceTable {
+  bf16* h[kMaxLayers];
+  float* z[kMaxLayers];
+  bf16* dz[kMaxLayers];
+};
+
+// A workgroup barrier that orders LDS alone: loads and stores of global memory stay in flight across
+// it (__syncthreads waits for them all).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The forward and the dZ chain of RT row tiles of 16 samples, Q = width / 64, 2 Q waves of 32 columns.
+// A layer costs its weights' way from L2 to the CU (131 KB at 256 wide, about 1 us) and its
+// epilogue's arithmetic: the weights are loaded once per workgroup straight to the lanes that use
+// them, all of a layer in flight together while the layer before ends, and one row tile per workgroup
+// spreads the epilogues over all CUs up to 8192 samples (512 workgroups, two per CU; 4096 samples 25 us,
+// 28 with two row tiles), past which two halve the weights' traffic.
+// The pre-activations wait for the backward in `zs`, each lane its own (read by the lane that wrote
+// them, from L2). Each product
+// accumulates over K in steps of 32 from zero and its epilogue is k_gemm's, so Z, H and dZ are the
+// layer-by-layer path's bits. At 4096 samples of 4 x 256 this takes 25 us (38 with
+// the weights read by rows), k_dw 11 and k_adam 6, where the 24 launches of the layer-by-layer step
+// took 260.
+// GATHER: sample i of the batch is idx[batch n + i] of x and t; else sample i.
+template <int Q, int RT, bool GATHER, bool TRACE>
+__global__ __launch_bounds__(128 * Q) void k_train(const float* __restrict__ x, const float* __restrict__ t, int n,
+                                                   int d_in, int d_out, const long long* __restrict__ idx,
+                                                   const StepState* __restrict__ st, const float* __restrict__ norm,
+                                                   const bf16* __restrict__ wb, const bf16* __restrict__ wbt,
+                                                   const float* __restrict__ params, TrainPlan P,
+                                                   bf16* __restrict__ packs, f32x4* __restrict__ zs,
+                                                   double* __restrict__ sum, TraceTable tr) {
+  constexpr int H = 64 * Q, kThreads = 128 * Q, ld = H + kPad, KS = H / kTileK, kIn = 32, ldz = kTileK + kPad, M = 16 * RT;
+  __shared__ __align__(16) bf16 act[M * ld];
+  __shared__ __align__(16) bf16 dzl[M * ldz];
+  const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+  const int row = lane % 16, g = lane / 16, kq = 8 * g, nb = 32 * wave;
+  const int m0 = static_cast<int>(blockIdx.x) * M;
+  // The tile of 32 samples, and with one row tile which half of its packs.
+  const long long tile = m0 / kPackTile;
+  const int half = RT == 1 ? m0 / 16 % 2 : 0;
+  const long long from = GATHER ? st->batch * n : 0;
+  bf16x8 w[KS][2];
+  f32x4 acc[RT][2];
+  auto load_w = [&](const bf16* W, int steps) {
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      if (k >= steps) break;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) w[k][j] = packed_operand(W, 2 * wave + j, k, steps);
+    }
+  };
+  auto product = [&](const bf16* a0, int lda, int steps) {
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      if (k >= steps) break;
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(a0 + (16 * i + row) * lda + kTileK * k + kq);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w[k][j], acc[i][j], 0, 0, 0);
+      }
+    }
+  };
+  // Column f of this lane's row tiles (acc's values after an epilogue): the tile's LDS rows for the
+  // next product, the pack (or the half of it that this row tile is), the traced tensor.
+  auto keep = [&](int f, const f32x4 (&v)[RT], long long at, bf16* traced) {
+    bf16x4 c[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      c[i] = __builtin_convertvector(v[i], bf16x4);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        act[(16 * i + 4 * g + r) * ld + f] = c[i][r];
+        if constexpr (TRACE) {
+          const int m = m0 + 16 * i + 4 * g + r;
+          if (m < n) traced[static_cast<long long>(m) * H + f] = c[i][r];
+        }
+      }
+    }
+    bf16* p = packs + at + ((tile * H + f) * 4 + g) * 8;
+    if constexpr (RT == 2) {
+      *reinterpret_cast<bf16x8*>(p) = __builtin_shufflevector(c[0], c[RT - 1], 0, 1, 2, 3, 4, 5, 6, 7);
+    } else {
+      *reinterpret_cast<bf16x4*>(p + 4 * half) = c[0];
+    }
+  };
+  load_w(wb + P.w(0), 1);
+  for (int i = tid; i < M * kIn; i += kThreads) {
+    const int r = i / kIn, c = i % kIn;
+    float v = 0.0f;
+    if (m0 + r < n && c < d_in) {
+      const long long s = GATHER ? idx[from + m0 + r] : m0 + r;
+      v = (x[s * d_in + c] - norm[c]) / norm[32 + c];
+    }
+    const bf16 b = static_cast<bf16>(v);
+    act[r * ld + c] = b;
+    if constexpr (TRACE) {
+      if (m0 + r < n) tr.h[0][static_cast<long long>(m0 + r) * kIn + c] = b;
+    }
+  }
+  for (int i = tid; i < M * ldz; i += kThreads) dzl[i] = static_cast<bf16>(0.0f);
+  lds_barrier();
+  // The packs of the first f_count features of an LDS tile of leading dimension lda.
+  auto pack_tile = [&](const bf16* a0, int lda, int f_count, long long at) {
+    for (int i = tid; i < 4 * RT * f_count; i += kThreads) {
+      const int f = i / (4 * RT), p = i / RT % 4, h = i % RT;
+      bf16x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = a0[(16 * h + 4 * p + r) * lda + f];
+      *reinterpret_cast<bf16x4*>(packs + at + ((tile * f_count + f) * 4 + p) * 8 + 4 * (half + h)) = v;
+    }
+  };
+  pack_tile(act, ld, kIn, P.h(0));
+  const int hidden = P.hidden;
+  f32x4* zl = zs + static_cast<long long>(blockIdx.x) * hidden * 2 * RT * kThreads + tid;
+  for (int l = 0; l < hidden; ++l) {
+    product(act, ld, l == 0 ? 1 : KS);
+    // The next product's weights, in flight over this layer's end: the next hidden layer's, or the
+    // transposed output weights the backward starts with.
+    if (l + 1 < hidden) {
+      load_w(wb + P.w(l + 1), KS);
+    } else {
+      load_w(wbt + P.wt(hidden), 1);
+    }
+    lds_barrier();  // every wave has read the layer's input: the tile takes its output
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int f = nb + 16 * j + row;
+      const float bf = params[P.b(l) + f];
+      f32x4 h[RT];
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        f32x4 z;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          z[r] = acc[i][j][r] + bf;
+          h[i][r] = silu(z[r]);
+          if constexpr (TRACE) {
+            const int m = m0 + 16 * i + 4 * g + r;
+            if (m < n) tr.z[l][static_cast<long long>(m) * H + f] = z[r];
+          }
+        }
+        zl[((2 * l + j) * RT + i) * kThreads] = z;
+      }
+      keep(f, h, P.h(l + 1), TRACE ? tr.h[l + 1] : nullptr);
+    }
+    lds_barrier();
+  }
+  // The output layer (16 columns): wave i the row tile i; then the loss and its gradient.
+  if (wave < RT) {
+    const bf16* W = wb + P.w(hidden);
+    f32x4 o{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(&act[(16 * wave + row) * ld + kTileK * k + kq]);
+      const bf16x8 b = packed_operand(W, 0, k, KS);
+      o = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, o, 0, 0, 0);
+    }
+    const float bo = params[P.b(hidden) + row];
+    float e2 = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int ml = 16 * wave + 4 * g + r, m = m0 + ml;
+      const float z = o[r] + bo;
+      float dv = 0.0f;
+      if (m < n && row < d_out) {
+        const long long s = GATHER ? idx[from + m] : m;
+        const float e = z - (t[s * d_out + row] - norm[64 + row]) / norm[96 + row];
+        e2 += e * e;
+        dv = 2.0f * e / (static_cast<float>(n) * d_out);
+      }
+      dzl[ml * ldz + row] = static_cast<bf16>(dv);
+      if constexpr (TRACE) {
+        if (m < n) {
+          tr.z[hidden][static_cast<long long>(m) * 16 + row] = z;
+          tr.dz[hidden][static_cast<long long>(m) * 16 + row] = static_cast<bf16>(dv);
+        }
+      }
+    }
+#pragma unroll
+    for (int o2 = 32; o2 > 0; o2 /= 2) e2 += __shfl_xor(e2, o2);
+    if (lane == 0) atomicAdd(sum, static_cast<double>(e2));
+  }
+  lds_barrier();
+  pack_tile(dzl, ldz, 16, P.dz(hidden));
+  // dZ_{l-1} = (dZ_l W_l) * silu'(Z_{l-1}).
+  for (int l = hidden; l > 0; --l) {
+    if (l == hidden) {
+      product(dzl, ldz, 1);
+    } else {
+      product(act, ld, KS);
+    }
+    if (l > 1) load_w(wbt + P.wt(l - 1), KS);
+    lds_barrier();
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int f = nb + 16 * j + row;
+      f32x4 dv[RT];
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const f32x4 z = zl[((2 * (l - 1) + j) * RT + i) * kThreads];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) dv[i][r] = acc[i][j][r] * silu_grad(z[r]);
+      }
+      keep(f, dv, P.dz(l - 1), TRACE ? tr.dz[l - 1] : nullptr);
+    }
+    lds_barrier();
+  }
+}
+
+// dW_l = dZ_l^T H_l (N_l x K_l) and db_l = the column sums of dZ_l for every layer, over the samples'
+// tiles of split blockIdx.x, into partial sums of their own (no atomics; summed in split
+// order by k_adam or k_sum_parts, so a step's gradients do not depend on the launch). A workgroup
+// has a 64 x 64 tile of one layer, each wave 32 x 32 of it, its operands read as the packs hold them,
+// one KB per 16 features and 32 samples, and stores its 16 x 16 products as it holds them, one KB each
+// (part_place): rows of a 64 x 64 tile are 1 KB apart, two of the L2's sixteen channels, and those
+// stores alone took 13 us.
+// With four tiles' packs in flight the loads' latency is hidden by few waves. Block 0 also counts the
+// step (the batch, Adam's step and bias corrections), after k_train has read it and before k_adam.
+__global__ __launch_bounds__(kThreads) void k_dw(const bf16* __restrict__ packs, TrainPlan P, int tiles, int per_split,
+                                                 float* __restrict__ part, long long np, StepState* st, float b1,
+                                                 float b2) {
+  if (st != nullptr && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+    st->batch += 1;
+    st->step += 1;
+    const float s = static_cast<float>(st->step);
+    st->c1 = 1.0f - powf(b1, s);
+    st->c2 = 1.0f - powf(b2, s);
+  }
+  // The layer and its 64 x 64 tile: q tiles of the first layer, q q of each hidden one, q of the last.
+  const int q = P.width / 64;
+  int l = 0, at = static_cast<int>(blockIdx.y);
+  if (at >= q) {
+    l = 1 + (at - q) / (q * q);
+    at = (at - q) % (q * q);
+  }
+  const int nf = l == P.hidden ? 1 : 4 * q, kf = l == 0 ? 2 : 4 * q;  // 16-feature fragments of N_l, K_l
+  const int kt = l == 0 ? 1 : q;
+  const long long ow = P.w(l), ob = P.b(l);
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int row = lane % 16, g = lane / 16;
+  const int n0 = 4 * (at / kt) + 2 * (wave / 2), k0 = 4 * (at % kt) + 2 * (wave % 2);  // fragments
+  if (n0 >= nf || k0 >= kf) return;
+  const bool n1 = n0 + 1 < nf, k1 = k0 + 1 < kf;
+  const bool bias = k0 == 0;
+  const bf16* A = packs + P.dz(l) + (16LL * n0 * 4 + 4 * row + g) * 8;
+  const bf16* B = packs + P.h(l) + (16LL * k0 * 4 + 4 * row + g) * 8;
+  const long long as = 16LL * nf * 32, bs = 16LL * kf * 32;  // values per sample tile
+  constexpr int kFrag = 16 * 32;
+  f32x4 acc[2][2];
+  float db[2] = {0.0f, 0.0f};
+  for (int i = 0; i < 2; ++i) {
+    for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  // A fragment past the layer's is read as the one before it, and its product not kept.
+  const long long a1 = n1 ? kFrag : 0, b1f = k1 ? kFrag : 0;
+  auto tiles_of = [&](int t, auto count) {
+    constexpr int kCount = decltype(count)::value;
+    bf16x8 a[kCount][2], b[kCount][2];
+#pragma unroll
+    for (int u = 0; u < kCount; ++u) {
+      const bf16* pa = A + (t + u) * as;
+      const bf16* pb = B + (t + u) * bs;
+      a[u][0] = *reinterpret_cast<const bf16x8*>(pa);
+      a[u][1] = *reinterpret_cast<const bf16x8*>(pa + a1);
+      b[u][0] = *reinterpret_cast<const bf16x8*>(pb);
+      b[u][1] = *reinterpret_cast<const bf16x8*>(pb + b1f);
+    }
+#pragma unroll
+    for (int u = 0; u < kCount; ++u) {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][i], b[u][j], acc[i][j], 0, 0, 0);
+      }
+    }
+    if (bias) {
+#pragma unroll
+      for (int u = 0; u < kCount; ++u) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+          for (int q8 = 0; q8 < 8; ++q8) db[i] += static_cast<float>(a[u][i][q8]);
+        }
+      }
+    }
+  };
+  int t = static_cast<int>(blockIdx.x) * per_split;
+  const int t1 = min(tiles, t + per_split);
+  constexpr int kAhead = 4;
+  for (; t + kAhead <= t1; t += kAhead) tiles_of(t, std::integral_constant<int, kAhead>{});
+  for (; t < t1; ++t) tiles_of(t, std::integral_constant<int, 1>{});
+  float* out = part + static_cast<long long>(blockIdx.x) * np;
+  for (int i = 0; i < 2; ++i) {
+    if (i == 1 && !n1) break;
+    for (int j = 0; j < 2; ++j) {
+      if (j == 1 && !k1) break;
+      reinterpret_cast<f32x4*>(out + ow)[((n0 + i) * kf + k0 + j) * 64 + lane] = acc[i][j];
+    }
+    if (bias) {
+      float v = db[i];
+      v += __shfl_xor(v, 16);
+      v += __shfl_xor(v, 32);
+      if (g == 0) out[ob + 16 * (n0 + i) + row] = v;
+    }
+  }
+}
+
+__global__ void k_sum_parts(const float* __restrict__ part, long long np, int splits, const int* __restrict__ order,
+                            float* __restrict__ g) {
+  const long long j = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (j < np) g[order[j]] = sum_parts(part, np, splits, j);
 }
 
 template <class T>
@@ -493,6 +895,40 @@ class Net {
     m2_ = Buf<float>(std::size_t(np_));
     wb_ = Buf<bf16>(std::size_t(np_));
     mask_ = Buf<unsigned char>(std::size_t(np_));
+    // The places of the packed copies (WeightCopies): every layer's weights, and the transposes of the
+    // layers after the first, the backward's operands.
+    std::vector<int2> at(std::size_t(np_), make_int2(-1, -1));
+    long long nt = 0;
+    for (int l = 0; l < nl; ++l) {
+      const int K = w_[std::size_t(l)], N = w_[std::size_t(l) + 1], ld = std::max(N, 32);
+      for (int n = 0; n < N; ++n) {
+        for (int k = 0; k < K; ++k) {
+          const long long i = woff_[std::size_t(l)] + static_cast<long long>(n) * K + k;
+          at[std::size_t(i)] = make_int2(static_cast<int>(woff_[std::size_t(l)] + pack_place(n, k, K / 32)),
+                                         l > 0 ? static_cast<int>(nt + pack_place(k, n, ld / 32)) : -1);
+        }
+      }
+      if (l > 0) nt += static_cast<long long>(K) * ld;
+    }
+    place_ = Buf<int2>(std::size_t(np_));
+    wp_ = Buf<bf16>(std::size_t(np_));
+    wt_ = Buf<bf16>(std::size_t(nt));
+    std::vector<int> order(static_cast<std::size_t>(np_));
+    const TrainPlan plan{layers, hidden, 0};
+    for (int l = 0; l < nl; ++l) {
+      const int K = w_[std::size_t(l)], N = w_[std::size_t(l) + 1];
+      for (int n = 0; n < N; ++n) {
+        for (int k = 0; k < K; ++k) {
+          order[std::size_t(plan.part_place(l, n, k))] = static_cast<int>(woff_[std::size_t(l)] + static_cast<long long>(n) * K + k);
+        }
+        const long long b = boff_[std::size_t(l)] + n;
+        order[std::size_t(b)] = static_cast<int>(b);
+      }
+    }
+    order_ = Buf<int>(std::size_t(np_));
+    check(hipMemcpy(order_.get(), order.data(), np_ * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy");
+    check(hipMemcpy(place_.get(), at.data(), np_ * sizeof(int2), hipMemcpyHostToDevice), "hipMemcpy");
+    check(hipMemset(wt_.get(), 0, std::size_t(nt) * sizeof(bf16)), "hipMemset");
     check(hipMemcpy(params_.get(), host.data(), np_ * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
     check(hipMemcpy(mask_.get(), mask.data(), np_, hipMemcpyHostToDevice), "hipMemcpy");
     check(hipMemset(m1_.get(), 0, np_ * sizeof(float)), "hipMemset");
@@ -556,9 +992,15 @@ class Net {
     Buf<float> xd(std::size_t(n) * d_in_), td(std::size_t(n) * d_out_);
     check(hipMemcpyAsync(xd.get(), x, std::size_t(n) * d_in_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
     check(hipMemcpyAsync(td.get(), t, std::size_t(n) * d_out_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
-    ensure(n);
+    ensure_loss();
     check(hipMemsetAsync(loss_sum_.get(), 0, sizeof(double), s_), "hipMemsetAsync");
-    backward(xd.get(), td.get(), n);
+    if (fused_training()) {
+      train_batch<false>(xd.get(), td.get(), n, nullptr);
+      k_sum_parts<<<cdiv(np_, 256), 256, 0, s_>>>(part_.get(), np_, splits_of(n), order_.get(), grads_.get());
+      check(hipGetLastError(), "k_sum_parts");
+    } else {
+      backward(xd.get(), td.get(), n);
+    }
     double sum = 0.0;
     check(hipMemcpyAsync(&sum, loss_sum_.get(), sizeof(double), hipMemcpyDeviceToHost, s_), "hipMemcpyAsync");
     check(hipStreamSynchronize(s_), "gradients");
@@ -577,8 +1019,19 @@ class Net {
     check(hipMemcpyAsync(xd.get(), x, std::size_t(n) * d_in_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
     check(hipMemcpyAsync(td.get(), t, std::size_t(n) * d_out_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
     ensure(n);
+    ensure_loss();
     check(hipMemsetAsync(loss_sum_.get(), 0, sizeof(double), s_), "hipMemsetAsync");
-    backward(xd.get(), td.get(), n);
+    if (fused_training()) {
+      TraceTable tr{};
+      for (std::size_t q = 0; q < std::size_t(nl); ++q) {
+        tr.h[q] = acts_[q].get();
+        tr.z[q] = z_[q].get();
+        tr.dz[q] = dz_[q].get();
+      }
+      train_batch<false>(xd.get(), td.get(), n, &tr);
+    } else {
+      backward(xd.get(), td.get(), n);
+    }
     const std::size_t l = static_cast<std::size_t>(layer);
     const std::size_t count = std::size_t(n) * std::size_t(what == 0 ? w_[l] : w_[l + 1]);
     if (what == 1) {
@@ -607,7 +1060,8 @@ class Net {
   float train(int epochs, int batch, float lr, uint64_t seed, double* seconds) {
     if (n_data_ < batch || batch < 64) throw std::invalid_argument("mlp: batch >= 64 and <= the data");
     const long long nb = n_data_ / batch;
-    Buf<float> bx(std::size_t(batch) * d_in_), bt(std::size_t(batch) * d_out_);
+    const bool fused = fused_training();
+    Buf<float> bx(fused ? 0 : std::size_t(batch) * d_in_), bt(fused ? 0 : std::size_t(batch) * d_out_);
     Buf<long long> idx(static_cast<std::size_t>(n_data_));
     std::vector<long long> order(static_cast<std::size_t>(n_data_));
     std::mt19937_64 rng(seed);
@@ -628,11 +1082,23 @@ class Net {
       std::shuffle(order.begin(), order.end(), rng);
       check(hipMemcpyAsync(idx.get(), order.data(), order.size() * sizeof(long long), hipMemcpyHostToDevice, s_),
             "hipMemcpyAsync");
-      ensure(batch);
+      if (fused) {
+        ensure_packs(batch);
+      } else {
+        ensure(batch);
+      }
+      ensure_loss();
       check(hipMemsetAsync(loss_sum_.get(), 0, sizeof(double), s_), "hipMemsetAsync");
       k_set_batch<<<1, 1, 0, s_>>>(state_.get(), 0);
       check(hipGetLastError(), "k_set_batch");
-      if (step_graph == nullptr) {
+      if (fused) {
+        // Three launches a step: plain ones keep ahead of the GPU (a graph of one step leaves 8 us
+        // between replays).
+        for (long long b = 0; b < nb; ++b) {
+          train_batch<true>(data_x_.get(), data_t_.get(), batch, nullptr, idx.get());
+          adam(lr, part_.get(), splits_of(batch), order_.get());
+        }
+      } else if (step_graph == nullptr) {
         // One step (gather of the state's batch, forward, loss, backward, Adam, next batch)
         // recorded once and replayed for every batch: its launches cost one graph launch.
         check(hipStreamBeginCapture(s_, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
@@ -642,7 +1108,8 @@ class Net {
                                                      data_t_.get(), d_out_, bx.get(), bt.get());
           check(hipGetLastError(), "k_gather");
           backward(bx.get(), bt.get(), batch);
-          adam(lr);
+          next_step();
+          adam(lr, grads_.get(), 1, nullptr);
         } catch (...) {
           (void)hipStreamEndCapture(s_, &g);
           if (g != nullptr) (void)hipGraphDestroy(g);
@@ -653,7 +1120,7 @@ class Net {
         (void)hipGraphDestroy(g);
         check(e, "hipGraphInstantiate");
       }
-      for (long long b = 0; b < nb; ++b) check(hipGraphLaunch(step_graph, s_), "hipGraphLaunch");
+      for (long long b = 0; b < nb && !fused; ++b) check(hipGraphLaunch(step_graph, s_), "hipGraphLaunch");
       double sum = 0.0;
       check(hipMemcpyAsync(&sum, loss_sum_.get(), sizeof(double), hipMemcpyDeviceToHost, s_), "hipMemcpyAsync");
       check(hipStreamSynchronize(s_), "train");
@@ -670,7 +1137,8 @@ class Net {
   }
 
   void adam_step(float lr) {
-    adam(lr);
+    next_step();
+    adam(lr, grads_.get(), 1, nullptr);
     check(hipStreamSynchronize(s_), "adam");
   }
 
@@ -689,10 +1157,10 @@ class Net {
       const float* nm = norm_.get();
       const float* pr = params_.get();
       switch (h / 64) {
-        case 1: launch_infer_rows<1>(infer_rows_, x, n, d_in_, d_out_, nm, wb_.get(), pr, L, y, s_); break;
-        case 2: launch_infer_rows<2>(infer_rows_, x, n, d_in_, d_out_, nm, wb_.get(), pr, L, y, s_); break;
-        case 3: launch_infer_rows<3>(infer_rows_, x, n, d_in_, d_out_, nm, wb_.get(), pr, L, y, s_); break;
-        default: launch_infer_rows<4>(infer_rows_, x, n, d_in_, d_out_, nm, wb_.get(), pr, L, y, s_); break;
+        case 1: launch_infer_rows<1>(infer_rows_, x, n, d_in_, d_out_, nm, wp_.get(), pr, L, y, s_); break;
+        case 2: launch_infer_rows<2>(infer_rows_, x, n, d_in_, d_out_, nm, wp_.get(), pr, L, y, s_); break;
+        case 3: launch_infer_rows<3>(infer_rows_, x, n, d_in_, d_out_, nm, wp_.get(), pr, L, y, s_); break;
+        default: launch_infer_rows<4>(infer_rows_, x, n, d_in_, d_out_, nm, wp_.get(), pr, L, y, s_); break;
       }
       check(hipGetLastError(), "k_infer");
       return;
@@ -733,7 +1201,7 @@ class Net {
   static constexpr int kInPad = 32, kOutPad = 16;
 
   void refresh_bf16() {
-    k_to_bf16<<<cdiv(np_, 256), 256, 0, s_>>>(params_.get(), np_, wb_.get());
+    k_to_bf16<<<cdiv(np_, 256), 256, 0, s_>>>(params_.get(), np_, copies());
     check(hipGetLastError(), "k_to_bf16");
     check(hipStreamSynchronize(s_), "refresh");
   }
@@ -750,7 +1218,85 @@ class Net {
       z_.emplace_back(std::size_t(n) * w_[l]);
       dz_.emplace_back(std::size_t(n) * w_[l]);
     }
+  }
+
+  void ensure_loss() {
     if (loss_sum_.size() == 0) loss_sum_ = Buf<double>(1);
+  }
+
+  // The fused training step's kernels are built for these widths; wider networks train layer by layer.
+  bool fused_training() const { return w_[1] <= 256 && layers() <= kMaxLayers; }
+
+  // Up to this many samples a workgroup takes one row tile.
+  static constexpr int kOneRowTile = 8192;
+  static int tiles_of(int n) { return cdiv(n, kPackTile); }
+  // Partial gradients of a batch: eight sample tiles each where that gives at most 8, one per XCD (at 56
+  // tiles of weights for four hidden layers of 256, 4096 samples then make 448 workgroups; 16 take the
+  // same 11 us and cost k_adam 1 more).
+  static int splits_of(int n) {
+    const int tiles = tiles_of(n), want = std::max(1, std::min(8, cdiv(tiles, 8)));
+    return cdiv(tiles, cdiv(tiles, want));
+  }
+
+  // The packs, pre-activations and partial gradients of batches of up to n samples.
+  void ensure_packs(int n) {
+    const int splits = splits_of(n);
+    if (splits > part_splits_) {
+      part_ = Buf<float>(std::size_t(splits) * std::size_t(np_));
+      part_splits_ = splits;
+    }
+    if (n <= pack_cap_) return;
+    const std::size_t rows = std::size_t(tiles_of(n)) * kPackTile;
+    const std::size_t hidden = w_.size() - 2;
+    packs_ = Buf<bf16>(rows * (kInPad + kOutPad + 2 * hidden * std::size_t(w_[1])));
+    zs_ = Buf<f32x4>(rows * hidden * std::size_t(w_[1]) / 4);
+    pack_cap_ = n;
+  }
+
+  // The forward, loss and gradients of one batch of device-resident samples (of `idx`'s batch of the
+  // state, with GATHER): the partial gradients into part_, the squared errors added to loss_sum_. With
+  // GATHER it also counts the step. No host synchronisation.
+  template <bool GATHER>
+  void train_batch(const float* x, const float* t, int n, const TraceTable* tr, const long long* idx = nullptr) {
+    ensure_packs(n);
+    const int tiles = tiles_of(n), width = w_[1], q = width / 64;
+    const TrainPlan plan{layers() - 1, width, static_cast<long long>(tiles) * kPackTile};
+    auto run = [&](auto quarter, auto row_tiles, auto traced) {
+      constexpr int Q = decltype(quarter)::value, RT = decltype(row_tiles)::value;
+      k_train<Q, RT, GATHER, decltype(traced)::value><<<tiles * (2 / RT), 128 * Q, 0, s_>>>(
+          x, t, n, d_in_, d_out_, idx, state_.get(), norm_.get(), wp_.get(), wt_.get(), params_.get(), plan,
+          packs_.get(), zs_.get(), loss_sum_.get(), tr != nullptr ? *tr : TraceTable{});
+    };
+    auto sized = [&](auto quarter, auto traced) {
+      if (n <= kOneRowTile) {
+        run(quarter, std::integral_constant<int, 1>{}, traced);
+      } else {
+        run(quarter, std::integral_constant<int, 2>{}, traced);
+      }
+    };
+    auto pick = [&](auto traced) {
+      switch (q) {
+        case 1: sized(std::integral_constant<int, 1>{}, traced); break;
+        case 2: sized(std::integral_constant<int, 2>{}, traced); break;
+        case 3: sized(std::integral_constant<int, 3>{}, traced); break;
+        default: sized(std::integral_constant<int, 4>{}, traced); break;
+      }
+    };
+    if constexpr (!GATHER) {
+      if (tr != nullptr) {
+        pick(std::true_type{});
+      } else {
+        pick(std::false_type{});
+      }
+    } else {
+      pick(std::false_type{});
+    }
+    check(hipGetLastError(), "k_train");
+    const int splits = splits_of(n);
+    const int weight_tiles = 2 * q + (plan.hidden - 1) * q * q;
+    k_dw<<<dim3(splits, weight_tiles), kThreads, 0, s_>>>(packs_.get(), plan, tiles, cdiv(tiles, splits), part_.get(), np_,
+                                                  GATHER ? state_.get() : nullptr, kBeta1, kBeta2);
+    check(hipGetLastError(), "k_dw");
   }
 
   template <bool TA, bool TB, int EPI>
@@ -812,15 +1358,21 @@ class Net {
     }
   }
 
-  void adam(float lr) {
-    const float b1 = 0.9f, b2 = 0.999f;
-    k_next_step<<<1, 1, 0, s_>>>(state_.get(), b1, b2);
+  WeightCopies copies() const { return {wb_.get(), wp_.get(), wt_.get(), place_.get()}; }
+
+  void next_step() {
+    k_next_step<<<1, 1, 0, s_>>>(state_.get(), kBeta1, kBeta2);
     check(hipGetLastError(), "k_next_step");
-    k_adam<<<cdiv(np_, 256), 256, 0, s_>>>(params_.get(), grads_.get(), m1_.get(), m2_.get(), mask_.get(), np_, lr, b1,
-                                            b2, 1e-8f, state_.get(), wb_.get());
+  }
+
+  // Adam's update of the counted step, by the sum of `splits` partial gradients.
+  void adam(float lr, const float* part, int splits, const int* order) {
+    k_adam<<<cdiv(np_, 256), 256, 0, s_>>>(params_.get(), part, splits, order, m1_.get(), m2_.get(), mask_.get(), np_, lr,
+                                           kBeta1, kBeta2, 1e-8f, state_.get(), copies());
     check(hipGetLastError(), "k_adam");
   }
 
+  static constexpr float kBeta1 = 0.9f, kBeta2 = 0.999f;
   int d_in_, d_out_;
   hipStream_t s_ = nullptr;
   std::vector<int> w_;
@@ -829,7 +1381,13 @@ class Net {
   Buf<float> params_, grads_, m1_, m2_, norm_;
   Buf<StepState> state_;
   Buf<double> loss_sum_;
-  Buf<bf16> wb_;
+  Buf<bf16> wb_, wp_, wt_;  // the BF16 weights by row, packed, and packed transposed
+  Buf<int2> place_;
+  Buf<int> order_;  // the parameter at each place of the partial gradients
+  Buf<bf16> packs_;
+  Buf<f32x4> zs_;
+  Buf<float> part_;
+  int pack_cap_ = 0, part_splits_ = 0;
   Buf<unsigned char> mask_;
   std::vector<Buf<bf16>> acts_, dz_;
   std::vector<Buf<float>> z_;

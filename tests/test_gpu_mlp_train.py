@@ -1,0 +1,71 @@
+"""The fused training step (one kernel for the forward, the loss and the backward's chain, one for every
+layer's gradients) where its tiles can go wrong: batches around the 16- and 32-sample tiles and around
+the switch between one and two row tiles per workgroup, every width it is built for and the layered
+path past them, one hidden layer and many, inputs and outputs that fill their padding; against the FP64
+oracle of the BF16 network, whose gradients the kernels' own roundings of the activations and of dZ
+leave within the bound below. And an epoch on whole batches against the same batches given one by one
+to gradients() and adam_step()."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from autan_amd.mlp import MLP
+from oracle import mlp_oracle as mo
+
+pytestmark = pytest.mark.gpu
+
+
+def data(n, d_in, d_out, seed):
+    rng = np.random.default_rng(seed)
+    x = rng.uniform(-1, 1, size=(n, d_in)).astype(np.float32)
+    t = np.stack([np.sin((j + 1) * x[:, j % d_in]) + x[:, (j + 2) % d_in] for j in range(d_out)], axis=1)
+    return x, t.astype(np.float32)
+
+
+@pytest.mark.parametrize("hidden,layers,d_in,d_out", [(64, 1, 7, 5), (128, 3, 1, 1), (192, 2, 32, 16), (256, 6, 7, 5),
+                                                      (320, 2, 7, 5)])
+@pytest.mark.parametrize("n", [1, 16, 17, 33, 8192, 8193])
+def test_gradients_at_the_tiles_edges(hidden, layers, d_in, d_out, n):
+    m = MLP(d_in, hidden, layers, d_out, seed=n)
+    x, t = data(n, d_in, d_out, n + 1)
+    m.fit_normalization(*data(2000, d_in, d_out, 5))
+    loss, g = m.gradients(x, t)
+    norm = [np.asarray(a, np.float64) for a in m.norm]
+    l_o, g_o = mo.loss_and_gradients(m.params(), m.widths(), x, t, norm, d_out, bf=True)
+    assert abs(loss - l_o) <= 1e-2 * l_o
+    # Each BF16 rounding of a layer (2^-9 of a value) enters the gradients below it once, forward and
+    # backward: 2 layers of them, uncorrelated, well under 3 % of the norm.
+    at = 0
+    w = m.widths()
+    for l in range(len(w) - 1):
+        k, nn = w[l], w[l + 1]
+        for size in (nn * k, nn):
+            seg = slice(at, at + size)
+            at += size
+            assert np.linalg.norm(g[seg] - g_o[seg]) <= 5e-2 * np.linalg.norm(g_o[seg]) + 1e-12, (l, size)
+    m.close()
+
+
+@pytest.mark.parametrize("hidden", [64, 256])
+def test_an_epoch_is_its_batches(hidden):
+    """One batch per epoch: the shuffle only permutes its samples, so the epochs' weights are those of
+    gradients() and adam_step() on the batch, but for the order of FP32 sums: the gradients' relative
+    difference of a few 2^-24 times the square root of the samples changes each Adam step (lr at most per
+    weight, whatever the gradient's size) only where the gradient itself is that small."""
+    n, steps, lr = 500, 4, 1e-3
+    x, t = data(n, 7, 5, 3)
+    a, b = MLP(7, hidden, 3, 5, seed=2), MLP(7, hidden, 3, 5, seed=2)
+    for m in (a, b):
+        m.fit_normalization(x, t)
+    p0 = a.params()
+    loss, _ = a.train(x, t, epochs=steps, batch=n, lr=lr, seed=1)
+    for _ in range(steps):
+        last, _ = b.gradients(x, t)
+        b.adam_step(lr)
+    pa, pb = a.params(), b.params()
+    moved = np.linalg.norm(pb - p0)
+    assert moved > 0 and np.abs(pa - p0).max() <= 1.01 * steps * lr
+    assert np.linalg.norm(pa - pb) <= 2e-2 * moved
+    assert loss == pytest.approx(last, rel=1e-3)
