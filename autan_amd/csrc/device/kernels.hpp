@@ -368,6 +368,12 @@ __global__ __launch_bounds__(kBlock) void k_grad(Dev<C> d) {
 // bounds and minima run in the same order as k_grad.
 // OCC > 0 asks the compiler for OCC waves per SIMD (registers capped accordingly): a variant for
 // the autotuner, same bits.
+// Bound by the stencil stream's bytes on a large mesh and by the loads' latency on a small one: kAhead
+// entries (and as many of the limiter's offsets) are in flight while the ones before are summed, the
+// first of them before the table is staged. With one entry ahead and nothing before the table: 308 us
+// on a 2.3M-cell channel in fp32 (1.25 GB; 270 now, 4.6 TB/s), 37 us on 33k cells (26), 57 us on 172k in
+// fp64 (50). Two entries ahead in fp64, whose four would cost a wave per SIMD (1.11 against 1.15 ms for
+// three steps of 172k cells); in fp32 two, four and six take the same time on large meshes.
 // A load of data read once per launch: with NT, marked non-temporal (streamed past the caches'
 // replacement, leaving them to the data other blocks read again); the same value either way.
 template <bool NT, class T>
@@ -381,6 +387,7 @@ __device__ __forceinline__ T stream_load(const T* p) {
 
 template <class C, bool LIMITER, int OCC = 0, bool NT = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1))) void k_grad_lds(Dev<C> d) {
+  constexpr int kAhead = std::is_same_v<C, float> ? 4 : 2;
   extern __shared__ __align__(16) unsigned char smem[];
   C* tab = reinterpret_cast<C*>(smem);
   const int blk = cell_block(d);
@@ -389,6 +396,32 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
   if (!case_active(d, cs) || !case_second(d, cs)) return;
   const Params<C>& pa = d.ptab[cs];
   const int t0 = d.tbeg[blk], tn = d.tbeg[blk + 1] - t0;
+  const int c = blk * kBlock + threadIdx.x;
+  const bool inside = c < d.nc;
+  const int lens = inside ? d.lens[c] : 0;
+  const int len = lens & 0xffff, ilen = lens >> 16;
+  // The wave's slice of the stencil stream: `longest` entries of 64 lanes (shorter cells' padded), so
+  // that loads past a lane's own entries need no branch; past the slice the last is read again.
+  const int slice = __builtin_amdgcn_readfirstlane(c) / kWave, lane = threadIdx.x % kWave;
+  const bool any = __builtin_amdgcn_readfirstlane(c) < d.nc;
+  const long long s0 = any ? d.soff[slice] : 0;
+  const int longest = any ? static_cast<int>((d.soff[slice + 1] - s0) / kWave) : 0;
+  // The entries' positions and weights, kAhead of them in flight while the ones before are summed
+  // (the first before the table is staged); the sums run in entry order.
+  int l_next[kAhead];
+  C w_next[kAhead][3];
+  auto entries = [&](int j0) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const long long k = s0 + static_cast<long long>(j0 + u < longest ? j0 + u : longest - 1) * kWave + lane;
+      l_next[u] = stream_load<NT>(d.sloc + k);
+      w_next[u][0] = stream_load<NT>(d.sw0 + k);
+      w_next[u][1] = stream_load<NT>(d.sw1 + k);
+      w_next[u][2] = stream_load<NT>(d.sw2 + k);
+    }
+  };
+  if (longest > 0) entries(0);
+  const W5<C> wc = inside ? load_w(d.prim, c) : W5<C>{};
   for (int j = threadIdx.x; j < tn; j += kBlock) {
     const int e = d.tent[t0 + j];
     const W5<C> w = e >= 0 ? load_w(d.prim, e) : load_w(d.prim_b, -e - 1);
@@ -399,9 +432,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
     tab[4 * tn + j] = w.p;
   }
   __syncthreads();
-  const int c = blk * kBlock + threadIdx.x;
-  if (c >= d.nc) return;
-  const W5<C> wc = load_w(d.prim, c);
+  if (!inside) return;
   const C wcv[5] = {wc.r, wc.u, wc.v, wc.w, wc.p};
   double acc[15];
 #pragma unroll
@@ -412,44 +443,48 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
     lo[q] = infinity<C>();
     hi[q] = -infinity<C>();
   }
-  const int lens = d.lens[c];
-  const int len = lens & 0xffff;
-  const long long base = d.soff[c / kWave] + (c % kWave);
-  // Entry j + 1's position and weights are loaded while entry j is summed (its loads' latency
-  // hidden behind the arithmetic); the sums run in entry order as before.
-  int l_next = 0;
-  C w0_next = C(0), w1_next = C(0), w2_next = C(0);
-  if (len > 0) {
-    l_next = stream_load<NT>(d.sloc + base);
-    w0_next = stream_load<NT>(d.sw0 + base);
-    w1_next = stream_load<NT>(d.sw1 + base);
-    w2_next = stream_load<NT>(d.sw2 + base);
-  }
-  for (int j = 0; j < len; ++j) {
-    const int l = l_next;
-    const C w0 = w0_next, w1 = w1_next, w2 = w2_next;
-    if (j + 1 < len) {
-      const long long k = base + static_cast<long long>(j + 1) * kWave;
-      l_next = stream_load<NT>(d.sloc + k);
-      w0_next = stream_load<NT>(d.sw0 + k);
-      w1_next = stream_load<NT>(d.sw1 + k);
-      w2_next = stream_load<NT>(d.sw2 + k);
-    }
+  for (int j0 = 0; j0 < longest; j0 += kAhead) {
+    int l[kAhead];
+    C w[kAhead][3];
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      const C wn = tab[i * tn + l];
-      const C dd = wn - wcv[i];
-      acc[3 * i] += static_cast<double>(dd * w0);
-      acc[3 * i + 1] += static_cast<double>(dd * w1);
-      acc[3 * i + 2] += static_cast<double>(dd * w2);
-      if (wn < lo[i]) lo[i] = wn;
-      if (wn > hi[i]) hi[i] = wn;
+    for (int u = 0; u < kAhead; ++u) {
+      l[u] = l_next[u];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) w[u][q] = w_next[u][q];
+    }
+    if (j0 + kAhead < longest) entries(j0 + kAhead);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      if (j0 + u >= len) continue;
+#pragma unroll
+      for (int i = 0; i < 5; ++i) {
+        const C wn = tab[i * tn + l[u]];
+        const C dd = wn - wcv[i];
+        acc[3 * i] += static_cast<double>(dd * w[u][0]);
+        acc[3 * i + 1] += static_cast<double>(dd * w[u][1]);
+        acc[3 * i + 2] += static_cast<double>(dd * w[u][2]);
+        if (wn < lo[i]) lo[i] = wn;
+        if (wn > hi[i]) hi[i] = wn;
+      }
     }
   }
   C out[20];
 #pragma unroll
   for (int q = 0; q < 15; ++q) out[q] = static_cast<C>(acc[q]);
   if constexpr (LIMITER) {
+    C r_next[kAhead][3];
+    const long long i0 = d.ioff[slice];
+    const int ilongest = static_cast<int>((d.ioff[slice + 1] - i0) / kWave);
+    auto offsets = [&](int j0) {
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        const long long k = i0 + static_cast<long long>(j0 + u < ilongest ? j0 + u : ilongest - 1) * kWave + lane;
+        r_next[u][0] = stream_load<NT>(d.ir0 + k);
+        r_next[u][1] = stream_load<NT>(d.ir1 + k);
+        r_next[u][2] = stream_load<NT>(d.ir2 + k);
+      }
+    };
+    if (ilongest > 0) offsets(0);
     C phi[5], eps2[5];
     const C vol = d.vol[c];
 #pragma unroll
@@ -459,29 +494,25 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
       phi[i] = infinity<C>();
       eps2[i] = pa.scale[i] * vol;
     }
-    const int ilen = lens >> 16;
-    const long long ib = d.ioff[c / kWave] + (c % kWave);
-    C r0_next = C(0), r1_next = C(0), r2_next = C(0);
-    if (ilen > 0) {
-      r0_next = stream_load<NT>(d.ir0 + ib);
-      r1_next = stream_load<NT>(d.ir1 + ib);
-      r2_next = stream_load<NT>(d.ir2 + ib);
-    }
-    for (int j = 0; j < ilen; ++j) {
-      const C r0 = r0_next, r1 = r1_next, r2 = r2_next;
-      if (j + 1 < ilen) {
-        const long long k = ib + static_cast<long long>(j + 1) * kWave;
-        r0_next = stream_load<NT>(d.ir0 + k);
-        r1_next = stream_load<NT>(d.ir1 + k);
-        r2_next = stream_load<NT>(d.ir2 + k);
-      }
+    for (int j0 = 0; j0 < ilongest; j0 += kAhead) {
+      C r[kAhead][3];
 #pragma unroll
-      for (int i = 0; i < 5; ++i) {
-        const C dd = out[3 * i] * r0 + out[3 * i + 1] * r1 + out[3 * i + 2] * r2;
-        const C dmax = hi[i] - wcv[i], dmin = lo[i] - wcv[i];
-        const C dp = dd > C(0.0) ? dmax : dmin;
-        const C v = (dp * dp + eps2[i] + C(2.0) * dd * dp) / (dp * dp + C(2.0) * dd * dd + dd * dp + eps2[i]);
-        if (v < phi[i]) phi[i] = v;
+      for (int u = 0; u < kAhead; ++u) {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) r[u][q] = r_next[u][q];
+      }
+      if (j0 + kAhead < ilongest) offsets(j0 + kAhead);
+#pragma unroll
+      for (int u = 0; u < kAhead; ++u) {
+        if (j0 + u >= ilen) continue;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+          const C dd = out[3 * i] * r[u][0] + out[3 * i + 1] * r[u][1] + out[3 * i + 2] * r[u][2];
+          const C dmax = hi[i] - wcv[i], dmin = lo[i] - wcv[i];
+          const C dp = dd > C(0.0) ? dmax : dmin;
+          const C v = (dp * dp + eps2[i] + C(2.0) * dd * dp) / (dp * dp + C(2.0) * dd * dd + dd * dp + eps2[i]);
+          if (v < phi[i]) phi[i] = v;
+        }
       }
     }
 #pragma unroll
