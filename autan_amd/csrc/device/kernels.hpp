@@ -597,6 +597,39 @@ struct StagedCells {
   }
 };
 
+// Whether a face's warp term with zero moments is zero in every component: its directions are zeros
+// then (gradient times zero), and so are their products with the mean state, unless one of the
+// factors is infinite or not a number, which this finds in the two sides' gradients and limiters, the
+// mean state, its |v|^2 and its enthalpy density (which bounds its momentum). Adding such a zero to a
+// flux could only turn -0 into +0, which no sum of fluxes from +0 shows. 98.5 % of a channel's faces
+// are flat: 47 multiply-adds instead of the term's 370 instructions, a third of the interior face's
+// arithmetic (172k cells in fp64: faces_rk 49.0 us before, 46.8 now; 2.3M in fp32: faces_first_rk 354 and
+// 340, faces_rk unchanged, bound by its gathers).
+template <bool SECOND, class C>
+__device__ __forceinline__ bool zero_warp(const W5<C>& w, const C* gl, const C* gr, C g, C pref) {
+  auto times_zero = [](C x, C sum) {
+    if constexpr (std::is_same_v<C, float>) {
+      return __builtin_fmaf(x, 0.0f, sum);
+    } else {
+      return __builtin_fma(x, 0.0, sum);
+    }
+  };
+  const C vv = dot(w.vel(), w.vel());
+  const C rh = g / (g - C(1.0)) * (w.p + pref) + C(0.5) * w.r * vv;
+  C z = times_zero(vv, times_zero(rh, times_zero(w.r, times_zero(w.p, C(0)))));
+  z = times_zero(w.u, times_zero(w.v, times_zero(w.w, z)));
+  if constexpr (SECOND) {
+    C zl = C(0), zr = C(0);  // two chains
+#pragma unroll
+    for (int q = 0; q < 20; ++q) {
+      zl = times_zero(gl[q], zl);
+      zr = times_zero(gr[q], zr);
+    }
+    z = z + (zl + zr);
+  }
+  return z == C(0);
+}
+
 // {flux}_face[_planar] and {flux}_boundary[_planar] (kernels/euler.py:687-1049) for the face `g`
 // (12 values, above): the area-weighted flux in C. The warp terms read the face's nine moments at
 // m[q * ms], or take zeros when the left index carries kFlatFace. With LAMBDA it also leaves the face's convective spectral radius
@@ -631,23 +664,25 @@ __device__ __forceinline__ F5<C> face_core(const Dev<C>& d, const Params<C>& pa,
 #pragma unroll
     for (int k = 0; k < 5; ++k) out.f[k] = area * fx.f[k];
     if constexpr (!PLANAR) {
-      C m[9];
-      if (flat) {
-#pragma unroll
-        for (int q = 0; q < 9; ++q) m[q] = C(0);
-      } else {
-#pragma unroll
-        for (int q = 0; q < 9; ++q) m[q] = m9[q * ms];
-      }
+      const W5<C> wm{C(0.5) * (fl.r + fr.r), C(0.5) * (fl.u + fr.u), C(0.5) * (fl.v + fr.v), C(0.5) * (fl.w + fr.w),
+                     C(0.5) * (fl.p + fr.p)};
       if constexpr (!SECOND) {
 #pragma unroll
         for (int q = 0; q < 20; ++q) gl[q] = gr[q] = C(0);
       }
-      const W5<C> wm{C(0.5) * (fl.r + fr.r), C(0.5) * (fl.u + fr.u), C(0.5) * (fl.v + fr.v), C(0.5) * (fl.w + fr.w),
-                     C(0.5) * (fl.p + fr.p)};
-      const F5<C> wp = warp(wm, gl, gl + 15, gr, gr + 15, m, pa.g, pa.pref);
+      if (!flat || !zero_warp<SECOND>(wm, gl, gr, pa.g, pa.pref)) {
+        C m[9];
+        if (flat) {
 #pragma unroll
-      for (int k = 0; k < 5; ++k) out.f[k] = out.f[k] + wp.f[k];
+          for (int q = 0; q < 9; ++q) m[q] = C(0);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 9; ++q) m[q] = m9[q * ms];
+        }
+        const F5<C> wp = warp(wm, gl, gl + 15, gr, gr + 15, m, pa.g, pa.pref);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) out.f[k] = out.f[k] + wp.f[k];
+      }
     }
   } else {
     const int b = -right - 1;
