@@ -1493,7 +1493,8 @@ class Stepper final : public StepperBase {
   // block its faces ascending, and for every incidence the LDS slot of its face with the cell's
   // side and whether the face is a boundary face.
   void build_slots(const int* cell_faces, const int* owner, const std::vector<int>& cfo) {
-    std::vector<int> cbeg{0}, sbeg{0}, sface;
+    std::vector<int> cbeg{0}, sface;
+    std::vector<int2> sbeg;
     sface.reserve(std::size_t(cfo.back()) / 2 + std::size_t(nc_));
     std::vector<unsigned short> islot(std::size_t(std::max(cfo.back(), 1)), 0);
     std::vector<int> mark(std::size_t(nf_), -1), faces;
@@ -1535,7 +1536,8 @@ class Stepper final : public StepperBase {
         }
       }
       sface.insert(sface.end(), faces.begin(), faces.end());
-      sbeg.push_back(static_cast<int>(sface.size()));
+      sbeg.push_back(make_int2(static_cast<int>(sface.size() - faces.size()), static_cast<int>(faces.size())));
+      sface.resize((sface.size() + kWave - 1) / kWave * kWave, -1);  // the next block's slots start a group
       cbeg.push_back(c);
     }
     face_blocks_ = static_cast<int>(cbeg.size()) - 1;
@@ -1543,7 +1545,7 @@ class Stepper final : public StepperBase {
     // Pad to the XCD-aware grid: the extra blocks hold no cell and no face.
     while (static_cast<int>(cbeg.size()) < xcd_grid(face_blocks_) + 1) {
       cbeg.push_back(nc_);
-      sbeg.push_back(sbeg.back());
+      sbeg.push_back(make_int2(static_cast<int>(sface.size()), 0));
       fcase.push_back(ncase_ - 1);
     }
     if (ncase_ == 1) fcbeg[1] = xcd_grid(face_blocks_);
@@ -2218,7 +2220,8 @@ class Stepper final : public StepperBase {
   RkStage<C> rk_{};  // the stage the next face launch updates (mode 0: none)
   Buffer<Small> small_;
   Buffer<unsigned long long> partial_;
-  Buffer<int> cbeg_, sbeg_;
+  Buffer<int> cbeg_;
+  Buffer<int2> sbeg_;
   std::vector<int> sface_host_;  // the faces of every slot, until the slot records are built
   bool stage_faces_ = false;     // fp32: the face kernel stages its block's cells in LDS
   // The gradient / face kernel built for at least this many waves per SIMD (0: the compiler's
