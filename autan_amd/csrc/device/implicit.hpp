@@ -11,9 +11,9 @@
 //   k_impl_relax(_run)        BlockMatrix::relax over the cells of one colour (a colour's cells share
 //                             no face, so they update together), or of a run of small colours;
 //   k_impl_multiply           BlockMatrix::multiply;
-//   k_impl_dot, k_impl_maxabs the GCR's inner products as exact sums and its largest entry
-//                             (EulerPhysics::owned_dot, owned_max_abs), the sums also fused into
-//                             the GCR's updates (k_impl_orth_dots, k_impl_advance_dot);
+//   k_impl_start, k_impl_scale_dot   the GCR's residual, its largest entry (owned_max_abs), scaled by it;
+//                             inner products as exact sums (EulerPhysics::owned_dot), fused into the
+//                             GCR's updates (k_impl_orth_dots, k_impl_advance_dot);
 //   k_impl_admissible         EulerPhysics::admissible_step: each cell's largest fraction of du that
 //                             keeps its density and pressure above half their values, the least over
 //                             the cells (an exact minimum of the FP64 values);
@@ -237,38 +237,48 @@ struct ImplRows {
 // place, five block columns, one value of the other cell per lane; the group's five values reach its
 // lanes by shuffles), since the sums that use them are one chain. A padding entry is a zero block
 // times zeros, which leaves r's bits (a sum from +0, or r - 0) as they are.
-constexpr int kSlots = 6;
+constexpr int kSlots = 3;
 
 template <bool ADD>
 __device__ __forceinline__ double impl_slots(const ImplRows& rows, int s, int lane, const double* __restrict__ offd,
                                              const double* x, double r) {
-  const bool on = lane < kSliceVec;
-  const int g = lane / 5, q = lane % 5, base = lane - q;
+  // No load stands behind a condition (the compiler moves one that does to its use): the idle lanes
+  // read the last row's, a slot past the slice the last slot's, and zeros take their place.
+  const int at = lane < kSliceVec ? lane : kSliceVec - 1;
+  const int g = at / 5, q = at % 5, base = lane - lane % 5;
   const int k1 = rows.slot[s + 1];
-  for (int k0 = rows.slot[s]; k0 < k1; k0 += kSlots) {
+  int next[kSlots];
+  // The places are read kSlots ahead, so that a long row's chain is one load per kSlots, not two.
+  auto places = [&](int k) {
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u) next[u] = rows.other[kSlice * (k + u < k1 ? k + u : k1 - 1) + g];
+  };
+  const int first = rows.slot[s];
+  if (first < k1) places(first);
+  for (int k0 = first; k0 < k1; k0 += kSlots) {
     int o[kSlots];
     double a[kSlots][5], xq[kSlots];
 #pragma unroll
     for (int u = 0; u < kSlots; ++u) {
-      const bool have = on && k0 + u < k1;
-      o[u] = have ? rows.other[kSlice * (k0 + u) + g] : -1;
+      o[u] = k0 + u < k1 ? next[u] : -1;
+      const double* block = offd + static_cast<long long>(kSliceBlock) * (k0 + u < k1 ? k0 + u : k1 - 1) + at;
 #pragma unroll
-      for (int j = 0; j < 5; ++j) {
-        a[u][j] = have ? offd[static_cast<long long>(kSliceBlock) * (k0 + u) + kSliceVec * j + lane] : 0.0;
-      }
+      for (int j = 0; j < 5; ++j) a[u][j] = block[kSliceVec * j];
     }
+    places(k0 + kSlots < k1 ? k0 + kSlots : first);
 #pragma unroll
-    for (int u = 0; u < kSlots; ++u) xq[u] = o[u] >= 0 ? x[5LL * o[u] + q] : 0.0;
+    for (int u = 0; u < kSlots; ++u) xq[u] = x[5LL * (o[u] >= 0 ? o[u] : 0) + q];
 #pragma unroll
     for (int u = 0; u < kSlots; ++u) {
-      if (k0 + u >= k1) break;
+      const double xu = o[u] >= 0 ? xq[u] : 0.0;
 #pragma unroll
       for (int j = 0; j < 5; ++j) {
-        const double xj = __shfl(xq[u], (base + j) % kWave);
+        const double xj = __shfl(xu, (base + j) % kWave);
+        const double aj = k0 + u < k1 ? a[u][j] : 0.0;
         if constexpr (ADD) {
-          r += a[u][j] * xj;
+          r += aj * xj;
         } else {
-          r -= a[u][j] * xj;
+          r -= aj * xj;
         }
       }
     }
@@ -279,22 +289,23 @@ __device__ __forceinline__ double impl_slots(const ImplRows& rows, int s, int la
 // BlockMatrix::relax of a slice's rows by one wave, lane 5 g + q row q of the g-th: x_c = D_c^-1 (b_c -
 // sum_f A_cf x_other). The group's five rows reach its lanes by shuffles for the inverse's product.
 // Bound by the blocks' bytes on a large colour and by the chain of loads (slot, place, value) on a
-// small one: the inverse, the right-hand side and six slots' blocks are in flight at once. With the
+// small one: the inverse, the right-hand side and three slots' blocks are in flight at once. With the
 // blocks row by row (each lane five consecutive values, a wave's loads 40 bytes apart) and one entry
 // in flight, two iterations of a 1.03M-cell channel took 54.1 ms where they now take 48.7 (the
-// relaxations 5.5 TB/s of blocks and values; two or three slots in flight 49.9 and 49.3 ms, each lane
-// reading the other cell's five values itself 54.2), a 39.5k-cell fp64 channel's 6.56 and 6.0 ms.
+// relaxations 5.5 TB/s of blocks and values; each lane reading the other cell's five values itself 54.2),
+// a 39.5k-cell fp64 channel's 6.56 and 6.0 ms.
 __device__ __forceinline__ void impl_relax_slice(const ImplRows& rows, int s, const double* __restrict__ offd,
                                                  const double* __restrict__ inverse, const double* __restrict__ b,
                                                  double* x) {
   const int lane = threadIdx.x % kWave;
   const bool on = lane < kSliceVec;
   const int base = lane - lane % 5;
-  const long long v = static_cast<long long>(kSliceVec) * s + lane;
+  const int at = on ? lane : kSliceVec - 1;  // the idle lanes repeat the last row's loads
+  const long long v = static_cast<long long>(kSliceVec) * s + at;
   double ip[5];
 #pragma unroll
-  for (int j = 0; j < 5; ++j) ip[j] = on ? inverse[static_cast<long long>(kSliceBlock) * s + kSliceVec * j + lane] : 0.0;
-  const double r = impl_slots<false>(rows, s, lane, offd, x, on ? b[v] : 0.0);
+  for (int j = 0; j < 5; ++j) ip[j] = inverse[static_cast<long long>(kSliceBlock) * s + kSliceVec * j + at];
+  const double r = impl_slots<false>(rows, s, lane, offd, x, b[v]);
   double sum = 0.0;
 #pragma unroll
   for (int j = 0; j < 5; ++j) sum += ip[j] * __shfl(r, (base + j) % kWave);
@@ -358,8 +369,10 @@ __global__ __launch_bounds__(kBlock) void k_impl_relax_start(int count, int n, c
 // colour is too small to fill the device.
 constexpr int kRelaxRunThreads = 1024;
 constexpr int kRelaxRunMax = 32;
-// Colours of at most this many slices (two passes of the run's workgroup) join a run.
-constexpr int kRelaxRunSlices = 2 * (kRelaxRunThreads / kWave);
+// Colours of at most this many slots join a run: their blocks (2.4 KB a slot) come into one CU, 64 bytes
+// a cycle, in 3 us or less, what a launch costs. A colour of 600 slots (1.03M-cell channel) took 13 us of
+// a run.
+constexpr int kRelaxRunSlots = 192;
 struct ImplRun {
   int first[kRelaxRunMax];
   int count[kRelaxRunMax];
@@ -389,12 +402,13 @@ __global__ __launch_bounds__(kBlock) void k_impl_multiply(ImplRows rows, int sli
   const int lane = threadIdx.x % kWave;
   const bool on = lane < kSliceVec;
   const int base = lane - lane % 5;
-  const long long v = static_cast<long long>(kSliceVec) * s + lane;
-  const double xq = on ? x[v] : 0.0;
+  const int at = on ? lane : kSliceVec - 1;
+  const long long v = static_cast<long long>(kSliceVec) * s + at;
+  const double xq = x[v];
   double r = 0.0;
 #pragma unroll
   for (int j = 0; j < 5; ++j) {
-    const double a = on ? diag[static_cast<long long>(kSliceBlock) * s + kSliceVec * j + lane] : 0.0;
+    const double a = diag[static_cast<long long>(kSliceBlock) * s + kSliceVec * j + at];
     r += a * __shfl(xq, (base + j) % kWave);
   }
   r = impl_slots<true>(rows, s, lane, offd, x, r);
@@ -461,16 +475,20 @@ __device__ __forceinline__ void impl_sum_flush(ImplSum* s, long long* const* wor
   }
 }
 
-// sum_i u_i v_i over m values as exact words (added into `words`, cleared beforehand): each product
-// rounded to FP64, then added exactly. Grid-stride.
-__global__ __launch_bounds__(kBlock) void k_impl_dot(const double* __restrict__ u, const double* __restrict__ v,
-                                                     long long m, long long* __restrict__ words) {
+// r /= s, s the number of these bits, and sum_i r_i r_i over the m values as exact words (added into
+// `words`, cleared beforehand): each product rounded to FP64, then added exactly. Grid-stride.
+__global__ __launch_bounds__(kBlock) void k_impl_scale_dot(double* __restrict__ r, long long m,
+                                                           const unsigned long long* __restrict__ scale_bits,
+                                                           long long* __restrict__ words) {
   __shared__ ImplSum acc[1];
   impl_sum_clear(acc[0]);
+  const double s = __longlong_as_double(static_cast<long long>(*scale_bits));
   __syncthreads();
   const long long stride = static_cast<long long>(gridDim.x) * kBlock;
   for (long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x; i < m; i += stride) {
-    impl_sum_add(acc[0], u[i] * v[i]);
+    const double v = r[i] / s;
+    r[i] = v;
+    impl_sum_add(acc[0], v * v);
   }
   long long* out[1] = {words};
   impl_sum_flush<1>(acc, out);
@@ -554,28 +572,19 @@ __global__ __launch_bounds__(kBlock) void k_impl_advance_dot(double* __restrict_
   impl_sum_flush<1>(acc, out);
 }
 
-// The largest |u_i| as the bits of a non-negative double (their integer order is their order);
-// a NaN entry leaves a NaN's bits, above every number's.
-__global__ __launch_bounds__(kBlock) void k_impl_maxabs(const double* __restrict__ u, long long m,
-                                                        unsigned long long* __restrict__ out) {
-  unsigned long long best = 0;
-  const long long stride = static_cast<long long>(gridDim.x) * kBlock;
-  for (long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x; i < m; i += stride) {
-    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(fabs(u[i])));
-    best = b > best ? b : best;
-  }
-  if (best != 0) atomicMax(out, best);
-}
+// What a solve leaves besides its sums: bits[0] the admissible fraction's minimum, bits[1] the residual's
+// largest entry, bits[2] the least cell with a singular diagonal block.
+constexpr int kImplBits = 3;
+__device__ __host__ inline int* impl_singular(unsigned long long* bits) { return reinterpret_cast<int*>(bits + 2); }
 
-// Clears n exact-sum words and sets *bits (the admissible fraction's minimum) to 1.0's bits,
-// *singular to INT32_MAX and the largest-entry bits to 0.
-__global__ void k_impl_clear(long long* __restrict__ words, int n, unsigned long long* __restrict__ bits,
-                             int* __restrict__ singular) {
+// Clears n exact-sum words and sets the fraction to 1.0's bits, the largest entry's to 0 and the
+// singular cell to INT32_MAX.
+__global__ void k_impl_clear(long long* __restrict__ words, int n, unsigned long long* __restrict__ bits) {
   for (int t = threadIdx.x; t < n; t += blockDim.x) words[t] = 0;
   if (threadIdx.x == 0) {
     bits[0] = static_cast<unsigned long long>(__double_as_longlong(1.0));
     bits[1] = 0;
-    *singular = INT32_MAX;
+    *impl_singular(bits) = INT32_MAX;
   }
 }
 
@@ -615,19 +624,21 @@ __global__ __launch_bounds__(kBlock) void k_impl_admissible(const double* __rest
     while (a >= kImplMinStep && !(impl_pressure(v0, dv, a, gamma) >= (1.0 - kImplMaxDecrease) * p)) a *= 0.5;
     key = static_cast<unsigned long long>(__double_as_longlong(a));
   }
+  // *bits starts at 1.0's, so a wave whose cells all take the full step has nothing to lower (one atomic
+  // per wave on that address took 188 us on 1.03M cells).
   key = wave_min(key);
-  if ((threadIdx.x % kWave) == 0 && key != ~0ULL) atomicMin(bits, key);
+  if ((threadIdx.x % kWave) == 0 && key < static_cast<unsigned long long>(__double_as_longlong(1.0))) atomicMin(bits, key);
 }
 
 // The Krylov operator's boundary term (EulerPhysics::add_boundary_gradient_term with
 // Euler::gradient_tangent, physics/src/euler_physics.cpp:1300-1320, physics/src/euler.cpp:1081-1119):
 // y += B v, the boundary faces' fluxes' derivative through the reconstruction's gradients, which
-// the assembled blocks drop. One thread per cell owning a boundary face (`cells`, ascending): the
+// the assembled blocks drop. Per cell owning a boundary face (`cells`, ascending): the
 // primitive tangents dW = dW/dq v of the cell and its stencil cells (the direction rounded to the
-// compute type, the products summed in it; k_impl_tangents, for every cell), the gradient's tangent sum_k (dW_k - dW_c) w_k (FP64
-// sums, boundary values held), then over its boundary faces in cell_faces order, where the
-// reconstruction did not fall back to the cell value, bnd_jac applied to phi (grad_tan . r), and on
-// warped slip and wall faces the wall-warp term's tangent phi_p M^T grad_tan p.
+// compute type, the products summed in it; k_impl_tangents, for the cells `near` lists), the gradient's
+// tangent sum_k (dW_k - dW_c) w_k (FP64 sums, boundary values held), then over its boundary faces in
+// cell_faces order, where the reconstruction did not fall back to the cell value, bnd_jac applied to
+// phi (grad_tan . r), and on warped slip and wall faces the wall-warp term's tangent phi_p M^T grad_tan p.
 // dwdu cell-major (25 c + 5 i + j), v by position (5 p + j).
 template <class C>
 __device__ __forceinline__ void impl_tangent(const double* __restrict__ dwdu, const double* __restrict__ v, long long c,
@@ -644,63 +655,82 @@ __device__ __forceinline__ void impl_tangent(const double* __restrict__ dwdu, co
   }
 }
 
-// Every cell's primitive tangent dW/dq v (impl_tangent), 5 x n in the compute type, for the
-// boundary term's stencils.
+// The primitive tangent dW/dq v (impl_tangent) of the listed cells, 5 consecutive values per cell in the
+// compute type, for the boundary term's stencils.
 template <class C>
 __global__ __launch_bounds__(kBlock) void k_impl_tangents(const double* __restrict__ dwdu, const double* __restrict__ v,
-                                                          const int* __restrict__ rank, int n, C* __restrict__ out) {
-  const int c = blockIdx.x * kBlock + threadIdx.x;
-  if (c >= n) return;
+                                                          const int* __restrict__ rank, const int* __restrict__ near,
+                                                          int count, C* __restrict__ out) {
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t >= count) return;
+  const int c = near[t];
   C dw[5];
   impl_tangent<C>(dwdu, v, c, rank[c], dw);
 #pragma unroll
-  for (int i = 0; i < 5; ++i) out[static_cast<long long>(i) * n + c] = dw[i];
+  for (int i = 0; i < 5; ++i) out[5LL * c + i] = dw[i];
 }
 
+// Five lanes per cell (12 cells per wave), lane i the tangents of variable i and then row i of the
+// faces' blocks, eight stencil entries in flight. The few thousand boundary cells leave most of the GPU
+// idle, so what counts is the chain of one cell's loads: with one thread per cell and one entry at a
+// time this took 57 us on 7.7k cells, 26 now.
 template <class C>
 __global__ __launch_bounds__(kBlock) void k_impl_bgrad(Dev<C> d, const int* __restrict__ cells, int count,
                                                        const C* __restrict__ tangents, const double* __restrict__ bj,
                                                        const int* __restrict__ rank, double* __restrict__ y) {
-  const int t = blockIdx.x * kBlock + threadIdx.x;
-  if (t >= count) return;
-  const int c = cells[t];
-  const long long n = d.nc;
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int g = lane / 5, i = lane % 5, base = lane - i;
+  const int t = (blockIdx.x * (kBlock / kWave) + wave) * kSlice + g;
+  // Lanes without a cell (60 .. 63, and past the list) repeat the last one: every lane shuffles.
+  const bool on = lane < kSliceVec && t < count;
+  const int c = cells[t < count ? t : count - 1];
   const Params<C>& pa = d.ptab[cell_case(d, c)];
-  C dwc[5];
-#pragma unroll
-  for (int i = 0; i < 5; ++i) dwc[i] = tangents[i * n + c];
-  double acc[15];
-#pragma unroll
-  for (int q = 0; q < 15; ++q) acc[q] = 0.0;
-  const long long base = d.soff[c / kWave] + (c % kWave);
+  const C dwc = tangents[5LL * c + i];
+  double acc[3] = {0.0, 0.0, 0.0};
+  const long long at = d.soff[c / kWave] + (c % kWave);
   const int len = d.slen[c];
-  for (int j = 0; j < len; ++j) {
-    const long long k = base + static_cast<long long>(j) * kWave;
-    const int e = d.sidx[k];
-    const C w0 = d.sw0[k], w1 = d.sw1[k], w2 = d.sw2[k];
-    C dwn[5] = {C(0), C(0), C(0), C(0), C(0)};
-    if (e >= 0) {
+  constexpr int kEntries = 8;
+  for (int j = 0; j < len; j += kEntries) {
+    int e[kEntries];
+    C w[kEntries][3], dwn[kEntries];
 #pragma unroll
-      for (int i = 0; i < 5; ++i) dwn[i] = tangents[i * n + e];
+    for (int u = 0; u < kEntries; ++u) {
+      const long long k = at + static_cast<long long>(j + u < len ? j + u : len - 1) * kWave;
+      e[u] = d.sidx[k];
+      w[u][0] = d.sw0[k];
+      w[u][1] = d.sw1[k];
+      w[u][2] = d.sw2[k];
     }
 #pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      const C dd = dwn[i] - dwc[i];
-      acc[3 * i] += static_cast<double>(dd * w0);
-      acc[3 * i + 1] += static_cast<double>(dd * w1);
-      acc[3 * i + 2] += static_cast<double>(dd * w2);
+    for (int u = 0; u < kEntries; ++u) {
+      const C v = tangents[5LL * (e[u] >= 0 ? e[u] : c) + i];
+      dwn[u] = e[u] >= 0 ? v : C(0);
+    }
+    // Past the cell's entries the last is read again and a zero added: a branch would have the
+    // compiler move the loads behind it.
+#pragma unroll
+    for (int u = 0; u < kEntries; ++u) {
+      const C dd = dwn[u] - dwc;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const double v = static_cast<double>(dd * w[u][q]);
+        acc[q] += j + u < len ? v : 0.0;
+      }
     }
   }
-  C gt[15];
+  C gt[3], gp[3];
 #pragma unroll
-  for (int q = 0; q < 15; ++q) gt[q] = static_cast<C>(acc[q]);
+  for (int q = 0; q < 3; ++q) gt[q] = static_cast<C>(acc[q]);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) gp[q] = __shfl(gt[q], base + 4 < kWave ? base + 4 : lane);  // the pressure's
   const W5<C> w = load_w(d.prim, c);
-  const C wc[5] = {w.r, w.u, w.v, w.w, w.p};
   C rec[20];
   load_rec(d.rec, c, rec);
   const C* gc = rec;
   const C* pc = rec + 15;
-  double dres[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+  const C phi = i == 0 ? pc[0] : i == 1 ? pc[1] : i == 2 ? pc[2] : i == 3 ? pc[3] : pc[4];
+  double dres = 0.0;
+  // Every lane of a group takes the same faces; groups of unlike counts meet no shuffle of another's.
   for (int k = d.cfo[c]; k < d.cfo[c + 1]; ++k) {
     const int f = d.inc[k] & 0x7fffffff;
     if (f < d.ni) continue;
@@ -710,59 +740,61 @@ __global__ __launch_bounds__(kBlock) void k_impl_bgrad(Dev<C> d, const int* __re
     const C r[3] = {g8[4], g8[5], g8[6]};
     const C d00 = gc[0] * r[0] + gc[1] * r[1] + gc[2] * r[2];
     const C d04 = gc[12] * r[0] + gc[13] * r[1] + gc[14] * r[2];
-    const bool fell_back = !((wc[0] + pc[0] * d00) > C(0.0) && (wc[4] + pc[4] * d04) + pa.pref > C(0.0));
+    const bool fell_back = !((w.r + pc[0] * d00) > C(0.0) && (w.p + pc[4] * d04) + pa.pref > C(0.0));
     if (fell_back) continue;
-    C dwf[5];
+    const C dwf = phi * (gt[0] * r[0] + gt[1] * r[1] + gt[2] * r[2]);
+    double s = 0.0;
 #pragma unroll
-    for (int i = 0; i < 5; ++i) dwf[i] = pc[i] * (gt[3 * i] * r[0] + gt[3 * i + 1] * r[1] + gt[3 * i + 2] * r[2]);
-#pragma unroll
-    for (int i = 0; i < 5; ++i) {
-      double s = 0.0;
-#pragma unroll
-      for (int j = 0; j < 5; ++j) s += bj[static_cast<long long>(5 * i + j) * d.nb + b] * static_cast<double>(dwf[j]);
-      dres[i] += s;
+    for (int j = 0; j < 5; ++j) {
+      const double v = static_cast<double>(__shfl(dwf, (base + j) % kWave));
+      s += bj[static_cast<long long>(5 * i + j) * d.nb + b] * v;
     }
+    dres += s;
     const int kind = d.bkind[b];
-    if (d.moment != nullptr && (kind == 2 || kind >= 5)) {
-      C m9[9];
-#pragma unroll
-      for (int q = 0; q < 9; ++q) m9[q] = d.moment[static_cast<long long>(q) * d.nf + f];
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        dres[1 + i] += static_cast<double>(pc[4] * (m9[i] * gt[12] + m9[3 + i] * gt[13] + m9[6 + i] * gt[14]));
-      }
+    if (d.moment != nullptr && (kind == 2 || kind >= 5) && i >= 1 && i <= 3) {
+      const long long n = d.nf;
+      const C* m = d.moment + static_cast<long long>(i - 1) * n + f;
+      dres += static_cast<double>(pc[4] * (m[0] * gp[0] + m[3 * n] * gp[1] + m[6 * n] * gp[2]));
     }
   }
-#pragma unroll
-  for (int i = 0; i < 5; ++i) y[5LL * rank[c] + i] += dres[i];
+  if (on) y[5LL * rank[c] + i] += dres;
 }
 
-// ---- the GCR's vector operations (solvers/src/gcr.cpp), m values each
+// ---- the solve's start and end, on the state's layout
 
-// y = -x, x as the residual holds it (value q of cell c at q n + c), y by position (m values; an
-// empty row's are 0).
-__global__ __launch_bounds__(kBlock) void k_impl_negate(const double* __restrict__ x, const int* __restrict__ cell,
-                                                        double* __restrict__ y, long long n, long long m) {
-  const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i >= m) return;
-  const int c = cell[i / 5];
-  y[i] = c >= 0 ? -x[(i % 5) * n + c] : 0.0;
+// r = -x and du = 0: x as the residual holds it (value q of cell c at q n + c), r and du by position (m
+// values; an empty row's are 0); and the largest |r_i| into *largest as the bits of a non-negative
+// double (their integer order is their order; a NaN's are above every number's), one atomic per block.
+__global__ __launch_bounds__(kBlock) void k_impl_start(const double* __restrict__ x, const int* __restrict__ cell,
+                                                       double* __restrict__ r, double* __restrict__ du, long long n,
+                                                       long long m, unsigned long long* __restrict__ largest) {
+  __shared__ unsigned long long wave_best[kBlock / kWave];
+  unsigned long long best = 0;
+  const long long stride = static_cast<long long>(gridDim.x) * kBlock;
+  for (long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x; i < m; i += stride) {
+    const int c = cell[i / 5];
+    const double v = c >= 0 ? -x[(i % 5) * n + c] : 0.0;
+    r[i] = v;
+    du[i] = 0.0;
+    const unsigned long long b = static_cast<unsigned long long>(__double_as_longlong(fabs(v)));
+    best = b > best ? b : best;
+  }
+  best = wave_max(best);
+  if (threadIdx.x % kWave == 0) wave_best[threadIdx.x / kWave] = best;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kBlock / kWave; ++w) best = wave_best[w] > best ? wave_best[w] : best;
+    if (best != 0) atomicMax(largest, best);
+  }
 }
 
-__global__ __launch_bounds__(kBlock) void k_impl_zero(double* __restrict__ x, long long m) {
-  const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i < m) x[i] = 0.0;
-}
-
-// r /= s (mode 0) or r *= s (mode 1)
-__global__ __launch_bounds__(kBlock) void k_impl_scale(double* __restrict__ r, long long m, double s, int mode) {
-  const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
-  if (i < m) r[i] = mode == 0 ? r[i] / s : r[i] * s;
-}
-
-// u += alpha du, u as the state holds it (value q of cell c at q n + c), du by position.
+// u += alpha du, alpha the number of these bits, unless it is below the least step; u as the state holds
+// it (value q of cell c at q n + c), du by position.
 __global__ __launch_bounds__(kBlock) void k_impl_update(double* __restrict__ u, const double* __restrict__ du,
-                                                        const int* __restrict__ rank, long long n, double alpha) {
+                                                        const int* __restrict__ rank, long long n,
+                                                        const unsigned long long* __restrict__ alpha_bits) {
+  const double alpha = __longlong_as_double(static_cast<long long>(*alpha_bits));
+  if (alpha < kImplMinStep) return;
   const long long i = static_cast<long long>(blockIdx.x) * kBlock + threadIdx.x;
   if (i < 5 * n) u[i] += alpha * du[5LL * rank[i % n] + i / n];
 }

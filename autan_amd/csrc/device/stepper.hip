@@ -310,7 +310,7 @@ class Stepper final : public StepperBase {
   void implicit_evaluate(double* norms, int* invalid) override {
     if (ncase_ != 1) throw std::invalid_argument("implicit step: one case");
     implicit_setup();
-    evaluate(norms, invalid);
+    enqueue_evaluate();
     const Dev<C> d = dev();
     launch("dwdu", [&] { k_dwdu<C, true><<<blocks(nc_), kBlock, 0, stream_>>>(d, u_.get(), jd_.get()); });
     launch("face_jacobian", [&] {
@@ -326,7 +326,7 @@ class Stepper final : public StepperBase {
           break;
       }
     });
-    check(hipStreamSynchronize(stream_), "implicit_evaluate");
+    finish(norms, invalid);
     have_jacobian_ = true;
     jac_second_ = second_;
   }
@@ -343,9 +343,8 @@ class Stepper final : public StepperBase {
     for (int q = 0; q < 5; ++q) report[q] = 0.0;
     const Dev<C> d = dev();
     const long long m = static_cast<long long>(kSliceVec) * slices_;
-    const int gm = static_cast<int>((m + kBlock - 1) / kBlock);
     dot_next_ = 0;
-    launch("impl_clear", [&] { k_impl_clear<<<1, 1024, 0, stream_>>>(words_.get(), static_cast<int>(words_.size()), bits_.get(), flag_.get());
+    launch("impl_clear", [&] { k_impl_clear<<<1, 1024, 0, stream_>>>(words_.get(), static_cast<int>(words_.size()), bits_.get());
     });
     if (ni_ > 0) {
       launch("impl_off", [&] {
@@ -358,13 +357,18 @@ class Stepper final : public StepperBase {
     });
     launch("impl_invert", [&] {
       k_impl_invert<<<blocks(kSlice * static_cast<long long>(slices_)), kBlock, 0, stream_>>>(
-          diag_.get(), ccells_.get(), kSlice * slices_, inv_.get(), flag_.get());
+          diag_.get(), ccells_.get(), kSlice * slices_, inv_.get(), impl_singular(bits_.get()));
     });
-    launch("impl_zero", [&] { k_impl_zero<<<gm, kBlock, 0, stream_>>>(du_.get(), m); });
-    launch("impl_negate", [&] { k_impl_negate<<<gm, kBlock, 0, stream_>>>(res_.get(), ccells_.get(), kr_.get(), nc_, m); });
-    int singular = INT32_MAX;
-    check(hipMemcpyAsync(&singular, flag_.get(), sizeof(int), hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
+    launch("impl_start", [&] {
+      k_impl_start<<<sum_grid(m), kBlock, 0, stream_>>>(res_.get(), ccells_.get(), kr_.get(), du_.get(), nc_, m,
+                                                        bits_.get() + 1);
+    });
+    const unsigned long long* hb = read_bits();
     check(hipStreamSynchronize(stream_), "implicit_solve");
+    int singular;
+    std::memcpy(&singular, hb + 2, sizeof singular);
+    double scale;
+    std::memcpy(&scale, hb + 1, sizeof scale);
     if (singular != INT32_MAX) {
       // A singular diagonal block: the solve failed (EulerPhysics::steady_step's domain_error).
       report[1] = std::numeric_limits<double>::quiet_NaN();
@@ -373,7 +377,7 @@ class Stepper final : public StepperBase {
       return;
     }
     int cycles = 0;
-    const double drop = gcr(m, gm, cycles);
+    const double drop = gcr(m, scale, cycles);
     report[0] = cycles;
     report[1] = drop;
     if (!(drop <= kImplFailure)) {
@@ -383,16 +387,15 @@ class Stepper final : public StepperBase {
     launch("impl_admissible", [&] {
       k_impl_admissible<<<blocks(nc_), kBlock, 0, stream_>>>(u_.get(), du_.get(), rank_.get(), nc_, sc_.gamma, bits_.get());
     });
-    unsigned long long abits = 0;
-    check(hipMemcpyAsync(&abits, bits_.get(), sizeof(abits), hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
+    launch("impl_update", [&] {
+      k_impl_update<<<blocks(5LL * nc_), kBlock, 0, stream_>>>(u_.get(), du_.get(), rank_.get(), nc_, bits_.get());
+    });
+    hb = read_bits();
     check(hipStreamSynchronize(stream_), "implicit_solve");
     double alpha;
-    std::memcpy(&alpha, &abits, sizeof alpha);
+    std::memcpy(&alpha, hb, sizeof alpha);
     report[2] = alpha;
-    if (alpha < kImplMinStep) return;
-    launch("impl_update", [&] { k_impl_update<<<blocks(5LL * nc_), kBlock, 0, stream_>>>(u_.get(), du_.get(), rank_.get(), nc_, alpha); });
-    prim_fresh_ = false;
-    check(hipStreamSynchronize(stream_), "implicit_solve");
+    if (alpha >= kImplMinStep) prim_fresh_ = false;
   }
 
   // EulerPhysics::worst_cell: the cell whose density or pressure the full step u + du lowers the
@@ -528,6 +531,8 @@ class Stepper final : public StepperBase {
     }
     nbo_ = static_cast<int>(bo.size());
     if (nbo_ > 0) bocells_.upload(bo, stream_);
+    // The cells whose tangents the boundary term reads: those and their stencils'.
+    if (nbo_ > 0) near_.upload(stencil_cells(bo), stream_);
     // Each interior face's entries in its two rows (slot times kSlice plus the row's place in its
     // slice), a row's entries in ascending face order, and the other cell's position of each.
     std::vector<int> rank(n);
@@ -555,7 +560,7 @@ class Stepper final : public StepperBase {
     rat_.upload(face_at, stream_);
     rank_.upload(rank, stream_);
     ccells_.upload(cells, stream_);
-    plan_relax();
+    plan_relax(slot);
     const std::size_t m = static_cast<std::size_t>(kSliceVec) * static_cast<std::size_t>(slices_);
     const std::size_t blk = static_cast<std::size_t>(kSliceBlock);
     jd_ = Buffer<double>(25 * n);
@@ -572,13 +577,35 @@ class Stepper final : public StepperBase {
     zs_ = Buffer<double>(m * kImplDirections);
     ws_ = Buffer<double>(m * kImplDirections);
     words_ = Buffer<long long>(std::size_t(kImplDots) * kWords + kImplHostWords);
-    bits_ = Buffer<unsigned long long>(2);
-    flag_ = Buffer<int>(1);
+    bits_ = Buffer<unsigned long long>(kImplBits);
     if (nbo_ > 0) tan_ = Buffer<C>(5 * n);
-    check(hipHostMalloc(reinterpret_cast<void**>(&host_words_), kImplHostWords * sizeof(long long), hipHostMallocDefault),
+    check(hipHostMalloc(reinterpret_cast<void**>(&host_words_), (kImplHostWords + kImplBits) * sizeof(long long),
+                        hipHostMallocDefault),
           "hipHostMalloc");
+    host_bits_ = reinterpret_cast<unsigned long long*>(host_words_ + kImplHostWords);
     check(hipStreamSynchronize(stream_), "implicit_setup");
     implicit_ready_ = true;
+  }
+
+  // The listed cells and the cells of their gradient stencils, ascending (from the device's stencil).
+  std::vector<int> stencil_cells(const std::vector<int>& list) {
+    std::vector<long long> soff(soff_.size());
+    std::vector<int> slen(slen_.size()), sidx(sidx_.size());
+    soff_.download(soff.data(), soff.size(), stream_);
+    slen_.download(slen.data(), slen.size(), stream_);
+    sidx_.download(sidx.data(), sidx.size(), stream_);
+    check(hipStreamSynchronize(stream_), "implicit_setup");
+    std::vector<int> out(list);
+    for (const int c : list) {
+      const long long base = soff[static_cast<std::size_t>(c / kWave)] + c % kWave;
+      for (int j = 0; j < slen[static_cast<std::size_t>(c)]; ++j) {
+        const int e = sidx[static_cast<std::size_t>(base + static_cast<long long>(j) * kWave)];
+        if (e >= 0) out.push_back(e);
+      }
+    }
+    std::sort(out.begin(), out.end());
+    out.erase(std::unique(out.begin(), out.end()), out.end());
+    return out;
   }
 
   // kImplSweeps symmetric sweeps on A z = b from z = 0: the colours in increasing, then decreasing
@@ -603,7 +630,7 @@ class Stepper final : public StepperBase {
     }
   }
 
-  // The sweeps' colour sequence as launches: a colour of more than kRelaxRunSlices slices is one
+  // The sweeps' colour sequence as launches: a colour of more than kRelaxRunSlots slots is one
   // launch over the device; consecutive smaller ones are one workgroup's run of phases.
   struct RelaxLaunch {
     int first = 0, count = 0;
@@ -624,7 +651,7 @@ class Stepper final : public StepperBase {
   // sweeps are bound by the blocks' bytes: on a 1.03M-cell channel 24.7M block reads instead of
   // 46.9M per direction, 7.3 GB instead of 13.6; two iterations of the implicit run there 74.2 ms
   // before, 54.1 ms with this plan (39.5k cells, fp64, second order: 7.23 and 6.56 ms).
-  void plan_relax() {
+  void plan_relax(const std::vector<int>& slot) {
     const int colours = static_cast<int>(colour_off_.size()) - 1;
     std::vector<std::array<int, 2>> order;  // first slice, slices
     for (int s = 0; s < kImplSweeps; ++s) {
@@ -639,7 +666,7 @@ class Stepper final : public StepperBase {
     relax_plan_.clear();
     for (const auto& [first, count] : order) {
       if (count == 0) continue;
-      const bool small = count <= kRelaxRunSlices;
+      const bool small = slot[static_cast<std::size_t>(first + count)] - slot[static_cast<std::size_t>(first)] <= kRelaxRunSlots;
       RelaxLaunch* last = relax_plan_.empty() ? nullptr : &relax_plan_.back();
       if (small && last != nullptr && last->run.phases > 0 && last->run.phases < kRelaxRunMax) {
         last->run.first[last->run.phases] = first;
@@ -663,33 +690,35 @@ class Stepper final : public StepperBase {
     }
   }
 
-  // Gcr::solve (solvers/src/gcr.cpp) on kr_ = -R into du_ = 0: returns the residual drop. The
+  // Grid of the kernels with exact sums: about 8 values per thread (a block's words cost it a fixed
+  // time), at most 1024 blocks.
+  static int sum_grid(long long m) {
+    return static_cast<int>(std::max<long long>(1, std::min<long long>(1024, m / (8LL * kBlock))));
+  }
+
+  // The solve's bits on their way to pinned memory (valid after the next synchronisation).
+  const unsigned long long* read_bits() {
+    check(hipMemcpyAsync(host_bits_, bits_.get(), kImplBits * sizeof(unsigned long long), hipMemcpyDeviceToHost, stream_),
+          "hipMemcpyAsync");
+    return host_bits_;
+  }
+
+  // Gcr::solve (solvers/src/gcr.cpp) on kr_ = -R, scale its largest entry, into du_ = 0: returns the residual drop. The
   // Gram-Schmidt and step coefficients are rounded and used on the device, each inner product fused
   // into the vector update before it (exact sums: the same bits in any order); the host reads (w, w)
   // and the words of (r, r) once per direction for the stopping rules, and takes every decision the
   // host loop takes, on the same values.
-  double gcr(long long m, int gm, int& cycles) {
+  double gcr(long long m, double scale, int& cycles) {
     // What the host reads of direction k: (w_k, w_k), which the next directions divide by, and the
     // words of (r, r), which the host rounds; direction 0's stand after the words of (r_0, r_0).
     auto ww_at = [](int k) { return kWords + k * (1 + kWords); };
     long long* hw = words_.get() + std::size_t(kImplDots) * kWords;
     auto ww_of = [&](int k) { return reinterpret_cast<double*>(hw + ww_at(k)); };
-    // Grid of the kernels with exact sums: about 8 values per thread (a block's words cost it a
-    // fixed time), at most 1024 blocks.
-    const int gd = static_cast<int>(std::max<long long>(1, std::min<long long>(1024, m / (8LL * kBlock))));
-    unsigned long long mbits = 0;
-    launch("impl_maxabs", [&] { k_impl_maxabs<<<gd, kBlock, 0, stream_>>>(kr_.get(), m, bits_.get() + 1); });
-    check(hipMemcpyAsync(&mbits, bits_.get() + 1, sizeof mbits, hipMemcpyDeviceToHost, stream_), "hipMemcpyAsync");
-    check(hipStreamSynchronize(stream_), "implicit_solve");
-    double scale;
-    std::memcpy(&scale, &mbits, sizeof scale);
+    const int gd = sum_grid(m);
     if (std::isnan(scale)) scale = std::numeric_limits<double>::infinity();
     if (!std::isfinite(scale)) return std::numeric_limits<double>::quiet_NaN();
     if (scale == 0.0) return 0.0;
-    launch("impl_scale", [&] { k_impl_scale<<<gm, kBlock, 0, stream_>>>(kr_.get(), m, scale, 0); });
-    {
-      launch("impl_dot", [&] { k_impl_dot<<<gd, kBlock, 0, stream_>>>(kr_.get(), kr_.get(), m, hw); });
-    }
+    launch("impl_scale_dot", [&] { k_impl_scale_dot<<<gd, kBlock, 0, stream_>>>(kr_.get(), m, bits_.get() + 1, hw); });
     double r0 = 0.0, rr = 0.0;
     for (int k = 0; k < kImplDirections; ++k) {
       double* z = zs_.get() + std::size_t(k) * std::size_t(m);
@@ -704,10 +733,12 @@ class Stepper final : public StepperBase {
       if (jac_second_ && nbo_ > 0) {
         const Dev<C> d = dev();
         launch("impl_tangents", [&] {
-          k_impl_tangents<C><<<blocks(nc_), kBlock, 0, stream_>>>(jd_.get(), z, rank_.get(), nc_, tan_.get());
+          k_impl_tangents<C><<<blocks(static_cast<long long>(near_.size())), kBlock, 0, stream_>>>(
+              jd_.get(), z, rank_.get(), near_.get(), static_cast<int>(near_.size()), tan_.get());
         });
+        constexpr int per = kBlock / kWave * kSlice;
         launch("impl_bgrad", [&] {
-          k_impl_bgrad<C><<<(nbo_ + kBlock - 1) / kBlock, kBlock, 0, stream_>>>(d, bocells_.get(), nbo_, tan_.get(),
+          k_impl_bgrad<C><<<(nbo_ + per - 1) / per, kBlock, 0, stream_>>>(d, bocells_.get(), nbo_, tan_.get(),
                                                                               jb_.get(), rank_.get(), w);
         });
       }
@@ -782,16 +813,17 @@ class Stepper final : public StepperBase {
 
   bool implicit_ready_ = false, have_jacobian_ = false, jac_second_ = false;
   int nbo_ = 0;  // cells owning a boundary face
-  Buffer<int> bocells_;
+  Buffer<int> bocells_, near_;
   int dot_next_ = 0;
   std::vector<int> colour_host_, colour_off_, colour_above_;
   int slices_ = 0;  // of the rows by position
-  Buffer<int> rslot_, rother_, rank_, ccells_, flag_;
+  Buffer<int> rslot_, rother_, rank_, ccells_;
   Buffer<int2> rat_;  // each interior face's two entries (owner's row, neighbour's row)
   Buffer<double> jd_, jf_, jb_, diag_, inv_, offd_, kr_, du_, zs_, ws_;
   Buffer<long long> words_;
   Buffer<unsigned long long> bits_;
   long long* host_words_ = nullptr;  // the pinned copy of the words and scalars the host reads
+  unsigned long long* host_bits_ = nullptr;  // after them, the solve's bits
   Buffer<C> tan_;  // the boundary term's primitive tangents
 
  public:
@@ -846,11 +878,15 @@ class Stepper final : public StepperBase {
   }
 
   void evaluate(double* residuals, int* invalid) override {
+    enqueue_evaluate();
+    finish(residuals, invalid);
+  }
+
+  void enqueue_evaluate() {
     clear();
     launch_prim(u_.get());
     residual_from_prim(true, 1.0, false);
     launch("check", [&] { k_check<C><<<cell_grid(), kBlock, 0, stream_>>>(dev(), u_.get()); });
-    finish(residuals, invalid);
   }
 
   void set_second_order(bool on) override {
