@@ -335,9 +335,12 @@ class SteadyCase {
 };
 
 // One steady run through the callbacks (EulerPhysics::device_step and the runtime's loop).
-// history (5 per iteration) and provisional (1 per iteration) may be null.
+// history (5 per iteration) and provisional (1 per iteration) may be null. `both`, where given, does a
+// provisional iteration's calls in one: the second-order norms into reported, then the first-order
+// step's.
+using Provisional = int (*)(void* ctx, double cfl, double reported[5], double residuals[5], int32_t* invalid);
 inline void run(const mxsteady_ops& ops, const mxsteady_options& o, mxsteady_result& out, double* history,
-                int32_t* provisional) {
+                int32_t* provisional, Provisional both = nullptr) {
   if (!ops.step || !ops.evaluate || !ops.set_second_order) throw std::invalid_argument("steady run: missing callback");
   SteadyCase sc(o);
   call(ops.set_second_order(ops.ctx, sc.second() ? 1 : 0), "set_second_order");
@@ -353,17 +356,20 @@ inline void run(const mxsteady_ops& ops, const mxsteady_options& o, mxsteady_res
     }
   }
   while (!sc.done()) {
-    double reported[kEq];
+    double reported[kEq], r[kEq];
     const bool prov = !sc.second();
-    if (prov) {
-      int32_t ignored = -1;
-      call(ops.set_second_order(ops.ctx, 1), "set_second_order");
-      call(ops.evaluate(ops.ctx, reported, &ignored), "evaluate");
-      call(ops.set_second_order(ops.ctx, 0), "set_second_order");
-    }
-    double r[kEq];
     int32_t invalid = -1;
-    call(ops.step(ops.ctx, o.cfl, r, &invalid), "step");
+    if (prov && both != nullptr) {
+      call(both(ops.ctx, o.cfl, reported, r, &invalid), "provisional step");
+    } else {
+      if (prov) {
+        int32_t ignored = -1;
+        call(ops.set_second_order(ops.ctx, 1), "set_second_order");
+        call(ops.evaluate(ops.ctx, reported, &ignored), "evaluate");
+        call(ops.set_second_order(ops.ctx, 0), "set_second_order");
+      }
+      call(ops.step(ops.ctx, o.cfl, r, &invalid), "step");
+    }
     sc.record(r, prov ? reported : nullptr, invalid, history, provisional);
     if (sc.switched()) call(ops.set_second_order(ops.ctx, 1), "set_second_order");
   }

@@ -138,6 +138,7 @@ class StepperBase {
                     int* invalid) = 0;
   virtual void evaluate(double* residuals, int* invalid) = 0;
   virtual void set_second_order(bool on) = 0;
+  virtual void provisional_step(double cfl, double* reported, double* residuals, int* invalid) = 0;
   virtual void set_boundary_data(const double* bc) = 0;
   virtual void set_source(const double* source) = 0;
   virtual void spectral_radius(double* lam) = 0;
@@ -209,8 +210,8 @@ class Stepper final : public StepperBase {
       bcase_.upload(bcase, stream_);
       cflags_host_.assign(std::size_t(ncase), 1 | (second_ ? 2 : 0));
       cflags_.upload(cflags_host_, stream_);
-      eflags_.upload(cflags_host_, stream_);
-      small_eval_ = Buffer<Small>(std::size_t(ncase));
+      eflags_host_ = cflags_host_;
+      eflags_.upload(eflags_host_, stream_);
     }
     build_topology(t);
     if (ncase > 1 && !fused_) throw std::invalid_argument("cases need the fused face kernel (blocks with too many faces)");
@@ -248,6 +249,7 @@ class Stepper final : public StepperBase {
     (void)hipStreamSynchronize(stream_);
     drop_graphs();
     if (host_small_ != nullptr) (void)hipHostFree(host_small_);
+    if (host_eval_ != nullptr) (void)hipHostFree(host_eval_);
     if (host_words_ != nullptr) (void)hipHostFree(host_words_);
     if (ev_in_ != nullptr) (void)hipEventDestroy(ev_in_);
     if (ev_out_ != nullptr) (void)hipEventDestroy(ev_out_);
@@ -892,8 +894,78 @@ class Stepper final : public StepperBase {
   void set_second_order(bool on) override {
     drop_graphs();
     second_ = on;
+    clear_records();
+  }
+
+  // Gradients and limiter zero (nothing to do where no gradient kernel ran since they were), in the
+  // stream's order.
+  void clear_records() {
+    if (!rec_written_) return;
     check(hipMemsetAsync(rec_.get(), 0, rec_.size() * sizeof(C), stream_), "hipMemsetAsync");
-    check(hipStreamSynchronize(stream_), "set_second_order");
+    rec_written_ = false;
+  }
+
+  // A provisional iteration of a steady run (a stepper at first order): the norms of R(u) at second
+  // order, as set_second_order(1), evaluate, set_second_order(0) give them, then one first-order step on
+  // local time steps; one wait for both, and u's primitives and boundary values formed once.
+  void provisional_step(double cfl, double* reported, double* residuals, int* invalid) override {
+    double h = 0.0;
+    if (ncase_ != 1) throw std::invalid_argument("provisional_step: one case");
+    if (!fused_) {  // the unfused kernels' norms have one place
+      int ignored = -1;
+      set_second_order(true);
+      evaluate(reported, &ignored);
+      set_second_order(false);
+      step(cfl, false, 0.0, true, residuals, &h, invalid);
+      return;
+    }
+    want_eval();
+    second_ = true;
+    eval_mode_ = true;
+    try {
+      clear();
+      if (!prim_fresh_) launch_prim(u_.get());
+      residual_from_prim(true, 1.0, false);
+    } catch (...) {
+      second_ = false;
+      eval_mode_ = false;
+      throw;
+    }
+    second_ = false;
+    eval_mode_ = false;
+    clear_records();
+    prim_fresh_ = true;  // the current buffer holds u's primitives
+    read_eval();
+    if (use_graph_) {
+      graph_step(cfl, true);
+    } else {
+      bstate_fresh_ = true;  // of the first residual alone (a graph's is recorded for any step)
+      enqueue_step(cfl, false, 0.0, true);
+    }
+    finish(residuals, invalid);
+    eval_norms(reported);
+  }
+
+  // A second-order evaluation's results: their place on the device, and on the way to the host.
+  void want_eval() {
+    const std::size_t n = std::size_t(ncase_);
+    if (small_eval_.size() == 0) small_eval_ = Buffer<Small>(n);
+    if (host_eval_ == nullptr) {
+      check(hipHostMalloc(reinterpret_cast<void**>(&host_eval_), sizeof(Small) * n, hipHostMallocDefault), "hipHostMalloc");
+    }
+  }
+  void read_eval() {
+    check(hipMemcpyAsync(host_eval_, small_eval_.get(), sizeof(Small) * std::size_t(ncase_), hipMemcpyDeviceToHost,
+                         stream_),
+          "hipMemcpyAsync");
+  }
+  void eval_norms(double* reported) const {
+    for (int cs = 0; cs < ncase_; ++cs) {
+      for (int k = 0; k < kSums; ++k) {
+        reported[kSums * cs + k] =
+            std::sqrt(exact_value(host_eval_[cs].words[k]) / double(case_cells_[std::size_t(cs)]));
+      }
+    }
   }
 
   void set_boundary_data(const double* bc) override {
@@ -958,9 +1030,12 @@ class Stepper final : public StepperBase {
     }
     if (n == 0) return;
     if (n > INT32_MAX / 3) throw std::invalid_argument("face_force: too many faces");
-    Buffer<int> list(static_cast<std::size_t>(n));
-    Buffer<double> out(3 * static_cast<std::size_t>(n));
-    face_force_into(faces, n, force, list.get(), out.get());
+    // The staging stays with the stepper, as large as its longest list (at most its boundary).
+    if (force_list_.size() < static_cast<std::size_t>(n)) {
+      force_list_ = Buffer<int>(static_cast<std::size_t>(n));
+      force_out_ = Buffer<double>(3 * static_cast<std::size_t>(n));
+    }
+    face_force_into(faces, n, force, force_list_.get(), force_out_.get());
   }
 
   // face_force with its staging in the device's static array: no allocation; at most
@@ -1007,11 +1082,11 @@ class Stepper final : public StepperBase {
     source_ = std::move(saved);
     const Dev<C> d = dev();
     launch("flux", [&] { launch_flux(d); });
-    Buffer<long long> words(std::size_t(kConsSums) * kWords);
-    std::vector<long long> zero(words.size(), 0), host(words.size());
-    words.upload(zero.data(), zero.size(), stream_);
-    launch("conservation", [&] { k_conservation<C><<<1024, kBlock, 0, stream_>>>(d, words.get()); });
-    words.download(host.data(), host.size(), stream_);
+    if (cons_words_.size() == 0) cons_words_ = Buffer<long long>(std::size_t(kConsSums) * kWords);
+    std::vector<long long> host(cons_words_.size());
+    check(hipMemsetAsync(cons_words_.get(), 0, cons_words_.size() * sizeof(long long), stream_), "hipMemsetAsync");
+    launch("conservation", [&] { k_conservation<C><<<1024, kBlock, 0, stream_>>>(d, cons_words_.get()); });
+    cons_words_.download(host.data(), host.size(), stream_);
     check(hipStreamSynchronize(stream_), "conservation");
     for (int i = 0; i < kConsSums; ++i) out[i] = exact_value(host.data() + std::size_t(i) * kWords);
   }
@@ -1183,12 +1258,10 @@ class Stepper final : public StepperBase {
       const std::size_t range = std::size_t(case_first_[std::size_t(k) + 1]) - first;
       if ((old & 1) && !(flags[k] & 1)) {
         // Both state buffers hold the frozen state, whichever the next step reads.
-        for (std::size_t q = 0; q < 5; ++q) {
-          const std::size_t at = q * std::size_t(nc_) + first;
-          check(hipMemcpyAsync(stage_.get() + at, u_.get() + at, range * sizeof(double), hipMemcpyDeviceToDevice,
-                               stream_),
-                "hipMemcpyAsync");
-        }
+        const std::size_t pitch = std::size_t(nc_) * sizeof(double);
+        check(hipMemcpy2DAsync(stage_.get() + first, pitch, u_.get() + first, pitch, range * sizeof(double), 5,
+                               hipMemcpyDeviceToDevice, stream_),
+              "hipMemcpy2DAsync");
       }
       if ((old & 2) && !(flags[k] & 2)) {
         check(hipMemsetAsync(rec_.get() + 20 * first, 0, 20 * range * sizeof(C), stream_), "hipMemsetAsync");
@@ -1202,14 +1275,19 @@ class Stepper final : public StepperBase {
 
   // Norms of R(u) at second order for the cases marked in `which` (the others skipped), then
   // those cases' gradients cleared: the residual a first-order start reports.
-  void batch_evaluate_second(const std::vector<int>& which, double* reported) {
+  // On the stream: read_eval's copy is complete once the step after it has been waited for.
+  void batch_evaluate_second(const std::vector<int>& which) {
+    want_eval();
     std::vector<int> ef(static_cast<std::size_t>(ncase_), 0);
     for (int k = 0; k < ncase_; ++k) ef[std::size_t(k)] = which[std::size_t(k)] ? 3 : 0;
-    eflags_.upload(ef.data(), ef.size(), stream_);
+    if (ef != eflags_host_) {
+      eflags_host_ = std::move(ef);
+      eflags_.upload(eflags_host_.data(), eflags_host_.size(), stream_);
+    }
     eval_mode_ = true;
     try {
       clear();
-      launch_prim(u_.get());
+      if (!prim_fresh_) launch_prim(u_.get());
       residual_from_prim(true, 1.0, false);
       launch("zero_rec", [&] { k_zero_rec<C><<<cell_grid(), kBlock, 0, stream_>>>(dev()); });
     } catch (...) {
@@ -1217,16 +1295,7 @@ class Stepper final : public StepperBase {
       throw;
     }
     eval_mode_ = false;
-    check(hipMemcpyAsync(host_small_, small_eval_.get(), sizeof(Small) * std::size_t(ncase_), hipMemcpyDeviceToHost,
-                         stream_),
-          "hipMemcpyAsync");
-    check(hipStreamSynchronize(stream_), "evaluate");
-    for (int cs = 0; cs < ncase_; ++cs) {
-      for (int k = 0; k < kSums; ++k) {
-        reported[kSums * cs + k] =
-            std::sqrt(exact_value(host_small_[cs].words[k]) / double(case_cells_[std::size_t(cs)]));
-      }
-    }
+    read_eval();
   }
 
   // Every case's steady run together: each case's first-order start, local time steps and
@@ -1262,8 +1331,9 @@ class Stepper final : public StepperBase {
         any_prov = any_prov || which[std::size_t(k)];
       }
       if (!any) break;
-      if (any_prov) batch_evaluate_second(which, rep.data());
+      if (any_prov) batch_evaluate_second(which);
       batch_step(o.cfl, true, r.data(), ts.data(), inv.data());
+      if (any_prov) eval_norms(rep.data());
       bool changed = false;
       for (int k = 0; k < ncase_; ++k) {
         auto& run = runs[std::size_t(k)];
@@ -1910,7 +1980,10 @@ class Stepper final : public StepperBase {
   // R(u)) also leaves the spectral radius, the time steps and the exact norms' words.
   void residual_from_prim(bool first = false, double cfl = 0.0, bool local = false) {
     const Dev<C> d = dev();
-    if (nb_ > 0) launch("bstate", [&] { k_bstate<C><<<blocks(nb_), kBlock, 0, stream_>>>(d); });
+    const bool have_bstate = bstate_fresh_;
+    bstate_fresh_ = false;
+    if (second_) rec_written_ = true;
+    if (nb_ > 0 && !have_bstate) launch("bstate", [&] { k_bstate<C><<<blocks(nb_), kBlock, 0, stream_>>>(d); });
     if (second_) {
       const std::size_t lds = std::size_t(max_table_) * 5 * sizeof(C);
       if (staged_ && sc_.limiter && grad_nt_) {
@@ -2202,6 +2275,9 @@ class Stepper final : public StepperBase {
 
   mxeuler_scheme sc_;
   Buffer<double> rb_;
+  Buffer<int> force_list_;      // the wall loads' staging
+  Buffer<double> force_out_;
+  Buffer<long long> cons_words_;  // the conservation check's sums
   hipEvent_t ev_in_ = nullptr, ev_out_ = nullptr;
   double area_scale_ = 0.0;
   hipStream_t stream_ = nullptr;
@@ -2216,8 +2292,12 @@ class Stepper final : public StepperBase {
   std::vector<Params<C>> ptab_host_;
   std::vector<int> cflags_host_;
   Buffer<int> eflags_;       // the flags of a second-order evaluation of some cases
+  std::vector<int> eflags_host_;
   Buffer<Small> small_eval_;  // its norms
   bool eval_mode_ = false;
+  Small* host_eval_ = nullptr;   // its pinned copy
+  bool rec_written_ = false;     // a gradient kernel ran since the records were cleared
+  bool bstate_fresh_ = false;    // the boundary values are the current primitives' (one residual)
   bool use_graph_ = false, graphs_valid_ = false, graph_local_ = false;
   double graph_cfl_ = 0.0;
   struct GraphEntry {
@@ -2696,6 +2776,14 @@ int steady_evaluate(void* ctx, double residuals[5], int32_t* invalid) {
   }
 }
 
+int steady_provisional(void* ctx, double cfl, double reported[5], double residuals[5], int32_t* invalid) {
+  return device_call([&] {
+    int inv = -1;
+    static_cast<mxeuler_stepper*>(ctx)->impl->provisional_step(cfl, reported, residuals, &inv);
+    *invalid = inv;
+  });
+}
+
 int steady_order(void* ctx, int32_t on) {
   try {
     static_cast<mxeuler_stepper*>(ctx)->impl->set_second_order(on != 0);
@@ -2713,7 +2801,7 @@ int mxeuler_steady(mxeuler_stepper* s, const mxsteady_options* options, mxsteady
     if (!s || !options || !result) throw std::invalid_argument("null argument");
     if (s->impl->ncase() != 1) throw std::invalid_argument("a batch runs with mxeuler_batch_steady");
     const mxsteady_ops ops{s, steady_step, steady_evaluate, steady_order};
-    mxe::steady::run(ops, *options, *result, history, provisional);
+    mxe::steady::run(ops, *options, *result, history, provisional, steady_provisional);
   });
 }
 

@@ -974,8 +974,10 @@ class Net {
 
   // Forward of n samples (host arrays, n x inputs -> n x outputs, physical units).
   void predict(const float* x, long long n, float* y) {
-    const long long chunk = 1 << 16;
-    Buf<float> xd(std::size_t(std::min(n, chunk) * d_in_)), yd(std::size_t(std::min(n, chunk) * d_out_));
+    // Device copies of at most kChunk samples at a time (48 MB with every input and output in use), kept.
+    constexpr long long kChunk = 1 << 18;
+    const long long chunk = std::min(n, kChunk);
+    Buf<float>&xd = host_x(chunk), &yd = host_t(chunk);
     for (long long at = 0; at < n; at += chunk) {
       const int m = static_cast<int>(std::min(chunk, n - at));
       check(hipMemcpyAsync(xd.get(), x + at * d_in_, std::size_t(m) * d_in_ * sizeof(float), hipMemcpyHostToDevice, s_),
@@ -989,7 +991,7 @@ class Net {
 
   // Loss and gradients (FP32, in parameter order) of one batch; grads may be null.
   float gradients(const float* x, const float* t, int n, float* grads) {
-    Buf<float> xd(std::size_t(n) * d_in_), td(std::size_t(n) * d_out_);
+    Buf<float>&xd = host_x(n), &td = host_t(n);
     check(hipMemcpyAsync(xd.get(), x, std::size_t(n) * d_in_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
     check(hipMemcpyAsync(td.get(), t, std::size_t(n) * d_out_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
     ensure_loss();
@@ -1048,8 +1050,11 @@ class Net {
 
   // Training data resident on the device; epochs of shuffled batches with Adam.
   void set_data(const float* x, const float* t, long long n) {
-    data_x_ = Buf<float>(std::size_t(n) * d_in_);
-    data_t_ = Buf<float>(std::size_t(n) * d_out_);
+    if (data_x_.size() != std::size_t(n) * d_in_) {
+      data_x_ = Buf<float>(std::size_t(n) * d_in_);
+      data_t_ = Buf<float>(std::size_t(n) * d_out_);
+      idx_ = Buf<long long>(std::size_t(n));
+    }
     check(hipMemcpy(data_x_.get(), x, std::size_t(n) * d_in_ * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
     check(hipMemcpy(data_t_.get(), t, std::size_t(n) * d_out_ * sizeof(float), hipMemcpyHostToDevice), "hipMemcpy");
     n_data_ = n;
@@ -1062,7 +1067,7 @@ class Net {
     const long long nb = n_data_ / batch;
     const bool fused = fused_training();
     Buf<float> bx(fused ? 0 : std::size_t(batch) * d_in_), bt(fused ? 0 : std::size_t(batch) * d_out_);
-    Buf<long long> idx(static_cast<std::size_t>(n_data_));
+    const Buf<long long>& idx = idx_;
     std::vector<long long> order(static_cast<std::size_t>(n_data_));
     std::mt19937_64 rng(seed);
     float last = 0.0f;
@@ -1199,6 +1204,16 @@ class Net {
 
  private:
   static constexpr int kInPad = 32, kOutPad = 16;
+
+  // Room for n samples' inputs, or targets or outputs, on the device.
+  Buf<float>& host_x(long long n) {
+    if (host_x_.size() < std::size_t(n) * d_in_) host_x_ = Buf<float>(std::size_t(n) * d_in_);
+    return host_x_;
+  }
+  Buf<float>& host_t(long long n) {
+    if (host_t_.size() < std::size_t(n) * d_out_) host_t_ = Buf<float>(std::size_t(n) * d_out_);
+    return host_t_;
+  }
 
   void refresh_bf16() {
     k_to_bf16<<<cdiv(np_, 256), 256, 0, s_>>>(params_.get(), np_, copies());
@@ -1395,6 +1410,8 @@ class Net {
   bool fused_ = true;
   int infer_rows_ = 128;  // the fastest tile on an MI355X (eight waves, 4 waves per SIMD)
   Buf<float> data_x_, data_t_;
+  Buf<long long> idx_;             // the epoch's order
+  Buf<float> host_x_, host_t_;     // device copies of a call's host samples, targets or outputs
   long long n_data_ = 0;
 };
 
