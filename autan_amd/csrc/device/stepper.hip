@@ -856,15 +856,31 @@ class Stepper final : public StepperBase {
     release(caller);
   }
 
+  // The kernels read the caller's state and write the caller's residual where they are (the primitives
+  // are formed from all of u before any of res is written, so the two may be one array): a copy of each
+  // would be a third of a small mesh's launches. A batch's inactive cases are not evaluated: theirs is the
+  // stepper's last residual, copied with the others'.
   void residual_device(const double* u, double* res, hipStream_t caller) override {
     prim_fresh_ = false;
     join(caller);
-    check(hipMemcpyAsync(stage_.get(), u, 5 * std::size_t(nc_) * sizeof(double), hipMemcpyDeviceToDevice, stream_),
-          "hipMemcpyAsync D2D");
-    launch_prim(stage_.get());
-    residual_from_prim();
-    check(hipMemcpyAsync(res, res_.get(), 5 * std::size_t(nc_) * sizeof(double), hipMemcpyDeviceToDevice, stream_),
-          "hipMemcpyAsync D2D");
+    if (ncase_ > 1) {
+      const std::size_t bytes = 5 * std::size_t(nc_) * sizeof(double);
+      check(hipMemcpyAsync(stage_.get(), u, bytes, hipMemcpyDeviceToDevice, stream_), "hipMemcpyAsync D2D");
+      launch_prim(stage_.get());
+      residual_from_prim();
+      check(hipMemcpyAsync(res, res_.get(), bytes, hipMemcpyDeviceToDevice, stream_), "hipMemcpyAsync D2D");
+      release(caller);
+      return;
+    }
+    launch_prim(u);
+    res_out_ = res;
+    try {
+      residual_from_prim();
+    } catch (...) {
+      res_out_ = nullptr;
+      throw;
+    }
+    res_out_ = nullptr;
     release(caller);
   }
 
@@ -1435,7 +1451,7 @@ class Stepper final : public StepperBase {
     d.prim_b = prim_b_.get();
     d.rec = rec_.get();
     d.fflux = fflux_.get();
-    d.res = res_.get();
+    d.res = res_out_ != nullptr ? res_out_ : res_.get();
     d.lam = lam_.get();
     d.dt = dt_.get();
     d.small = small_.get();
@@ -2297,6 +2313,7 @@ class Stepper final : public StepperBase {
   bool eval_mode_ = false;
   Small* host_eval_ = nullptr;   // its pinned copy
   bool rec_written_ = false;     // a gradient kernel ran since the records were cleared
+  double* res_out_ = nullptr;    // where a residual goes other than res_ (during one call)
   bool bstate_fresh_ = false;    // the boundary values are the current primitives' (one residual)
   bool use_graph_ = false, graphs_valid_ = false, graph_local_ = false;
   double graph_cfl_ = 0.0;

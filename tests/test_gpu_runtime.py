@@ -164,3 +164,23 @@ def test_device_resident_calls_give_the_host_calls_bits(policy):
         for a in (u, out, res, out0):
             a.free()
         s.destroy()
+
+
+@pytest.mark.parametrize("policy", ["fp64", "fp32+acc64"])
+@pytest.mark.parametrize("n", [1, 7])
+def test_a_residual_in_place_of_its_state_is_the_host_calls(policy, n):
+    """residual_device reads the caller's state and writes the caller's array directly: also where the
+    two are one array, on meshes of one cell block and of a ragged ninth."""
+    from hipmem import DeviceArray
+
+    case = cases.tets_case(n)
+    with DeviceStepper(case.mesh, case.scheme, policy, case.bc_kind, case.bc, case.source) as dev:
+        want = dev.residual(case.u)
+        a = DeviceArray(5 * case.mesh.n_cells)
+        try:
+            for _ in range(2):
+                a.copy_from(case.u)
+                dev.residual_device(a.ptr, a.ptr)
+                np.testing.assert_array_equal(a.numpy(), want)
+        finally:
+            a.free()
