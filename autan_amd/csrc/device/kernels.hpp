@@ -565,8 +565,7 @@ __device__ __forceinline__ C* slot_part(C* srec, long long sl, int part) {
 }
 
 // A slot record's left index with its sign bit set: the face's nine moments are all +0 (bit for
-// bit), so the warp terms take zeros in registers instead of reading them; the same values, so
-// the same bits. Left indices are cells, never negative otherwise.
+// bit), so the warp terms are left out where zero_warp finds them zero, or take zeros for the moments; the same bits. Left indices are cells, never negative otherwise.
 constexpr unsigned kFlatFace = 0x80000000u;
 
 template <class C>
@@ -644,7 +643,8 @@ __device__ __forceinline__ bool zero_warp(const W5<C>& w, const C* gl, const C* 
 
 // {flux}_face[_planar] and {flux}_boundary[_planar] (kernels/euler.py:687-1049) for the face `g`
 // (12 values, above): the area-weighted flux in C. The warp terms read the face's nine moments at
-// m[q * ms], or take zeros when the left index carries kFlatFace. With LAMBDA it also leaves the face's convective spectral radius
+// m[q * ms], or are left out when the left index carries kFlatFace (where zero_warp finds that they
+// would be zeros). With LAMBDA it also leaves the face's convective spectral radius
 // (kernels/euler.py:1091-1112) as each side takes it: lam[0] = max(s_owner, s_other) A for the
 // owner, lam[1] = max(s_other, s_owner) A for the neighbour, s = |v . n| + c of the cells' (not
 // reconstructed) primitives and of the boundary state.

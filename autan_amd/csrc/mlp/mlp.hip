@@ -4,7 +4,8 @@
 //
 // Layout: samples are rows. Layer l maps K_l inputs to N_l outputs with weights W_l stored N_l x K_l
 // (row n holds the weights into output n), so every operand of the forward product is read along
-// K. The input width is padded to 32 and the output width to 16 with zero weights.
+// K; beside the FP32 masters the BF16 weights are packed as the matrix cores read them (1 KB per 16
+// outputs x 32 inputs) for the fused kernels. The input width is padded to 32 and the output width to 16 with zero weights.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -184,3 +184,31 @@ def test_a_residual_in_place_of_its_state_is_the_host_calls(policy, n):
                 np.testing.assert_array_equal(a.numpy(), want)
         finally:
             a.free()
+
+
+@pytest.mark.parametrize("policy", ["fp64", "fp32+acc64"])
+def test_a_residual_between_evaluation_and_solve_is_the_host_calls(policy):
+    """The solve reads the stepper's last residual: a residual_device before it leaves the one a host
+    residual would."""
+    from hipmem import DeviceArray
+
+    case = cases.tets_case(3)
+    u = 0.99 * case.u
+    with DeviceStepper(case.mesh, case.scheme, policy, case.bc_kind, case.bc, case.source) as dev:
+        a = DeviceArray(5 * case.mesh.n_cells)
+        try:
+            states = []
+            for device in (False, True):
+                dev.upload(case.u)
+                dev.implicit_evaluate()
+                if device:
+                    a.copy_from(u)
+                    dev.residual_device(a.ptr, a.ptr)
+                    np.testing.assert_array_equal(a.numpy(), want)
+                else:
+                    want = dev.residual(u).reshape(-1)
+                dev.implicit_solve(10.0)
+                states.append(dev.download())
+            np.testing.assert_array_equal(states[1], states[0])
+        finally:
+            a.free()
