@@ -13,6 +13,7 @@
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <random>
 #include <stdexcept>
 #include <string>
@@ -975,10 +976,9 @@ class Net {
 
   // Forward of n samples (host arrays, n x inputs -> n x outputs, physical units).
   void predict(const float* x, long long n, float* y) {
-    // Device copies of at most kChunk samples at a time (48 MB with every input and output in use), kept.
-    constexpr long long kChunk = 1 << 18;
     const long long chunk = std::min(n, kChunk);
-    Buf<float>&xd = host_x(chunk), &yd = host_t(chunk);
+    Staging staging(*this, chunk);
+    const Buf<float>&xd = staging.x(), &yd = staging.t();
     for (long long at = 0; at < n; at += chunk) {
       const int m = static_cast<int>(std::min(chunk, n - at));
       check(hipMemcpyAsync(xd.get(), x + at * d_in_, std::size_t(m) * d_in_ * sizeof(float), hipMemcpyHostToDevice, s_),
@@ -988,11 +988,13 @@ class Net {
             "hipMemcpyAsync");
       check(hipStreamSynchronize(s_), "predict");
     }
+    staging.keep();
   }
 
   // Loss and gradients (FP32, in parameter order) of one batch; grads may be null.
   float gradients(const float* x, const float* t, int n, float* grads) {
-    Buf<float>&xd = host_x(n), &td = host_t(n);
+    Staging staging(*this, n);
+    const Buf<float>&xd = staging.x(), &td = staging.t();
     check(hipMemcpyAsync(xd.get(), x, std::size_t(n) * d_in_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
     check(hipMemcpyAsync(td.get(), t, std::size_t(n) * d_out_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
     ensure_loss();
@@ -1007,6 +1009,7 @@ class Net {
     double sum = 0.0;
     check(hipMemcpyAsync(&sum, loss_sum_.get(), sizeof(double), hipMemcpyDeviceToHost, s_), "hipMemcpyAsync");
     check(hipStreamSynchronize(s_), "gradients");
+    staging.keep();
     const float loss = static_cast<float>(sum / (static_cast<double>(n) * d_out_));
     if (grads != nullptr) check(hipMemcpy(grads, grads_.get(), np_ * sizeof(float), hipMemcpyDeviceToHost), "hipMemcpy");
     return loss;
@@ -1206,15 +1209,40 @@ class Net {
  private:
   static constexpr int kInPad = 32, kOutPad = 16;
 
-  // Room for n samples' inputs, or targets or outputs, on the device.
-  Buf<float>& host_x(long long n) {
-    if (host_x_.size() < std::size_t(n) * d_in_) host_x_ = Buf<float>(std::size_t(n) * d_in_);
-    return host_x_;
-  }
-  Buf<float>& host_t(long long n) {
-    if (host_t_.size() < std::size_t(n) * d_out_) host_t_ = Buf<float>(std::size_t(n) * d_out_);
-    return host_t_;
-  }
+  // Samples predict takes to the device at a time.
+  static constexpr long long kChunk = 1 << 18;
+
+  // A call's device copies of n host samples: their inputs, and their targets or outputs. The call
+  // has them to itself: another one at the same time (mxmlp_predict may be called from several host
+  // threads) finds none kept and allocates its own, as every call would. One pair of at most kChunk
+  // samples (48 MB with every input and output in use) is kept between calls, for its two
+  // allocations and frees (83,300 predictions: 293 us with them, 250 without).
+  class Staging {
+   public:
+    Staging(Net& net, long long n) : net_(net) {
+      {
+        const std::lock_guard<std::mutex> lock(net_.staging_mutex_);
+        std::swap(x_, net_.staging_x_);
+        std::swap(t_, net_.staging_t_);
+      }
+      if (x_.size() < std::size_t(n) * net_.d_in_) x_ = Buf<float>(std::size_t(n) * net_.d_in_);
+      if (t_.size() < std::size_t(n) * net_.d_out_) t_ = Buf<float>(std::size_t(n) * net_.d_out_);
+    }
+    Buf<float>& x() { return x_; }
+    Buf<float>& t() { return t_; }
+    // Given back for a later call, the call's work on the stream being done (a call that throws frees them).
+    void keep() {
+      if (x_.size() > std::size_t(kChunk) * net_.d_in_ || t_.size() > std::size_t(kChunk) * net_.d_out_) return;
+      const std::lock_guard<std::mutex> lock(net_.staging_mutex_);
+      if (net_.staging_x_.size() >= x_.size()) return;  // another call's, as large
+      std::swap(x_, net_.staging_x_);
+      std::swap(t_, net_.staging_t_);
+    }
+
+   private:
+    Net& net_;
+    Buf<float> x_, t_;
+  };
 
   void refresh_bf16() {
     k_to_bf16<<<cdiv(np_, 256), 256, 0, s_>>>(params_.get(), np_, copies());
@@ -1412,7 +1440,8 @@ class Net {
   int infer_rows_ = 128;  // the fastest tile on an MI355X (eight waves, 4 waves per SIMD)
   Buf<float> data_x_, data_t_;
   Buf<long long> idx_;             // the epoch's order
-  Buf<float> host_x_, host_t_;     // device copies of a call's host samples, targets or outputs
+  std::mutex staging_mutex_;
+  Buf<float> staging_x_, staging_t_;  // the pair kept between calls (Staging)
   long long n_data_ = 0;
 };
 

@@ -27,7 +27,9 @@ int mxmlp_set_normalization(mxmlp* h, const float* in_mean, const float* in_scal
                             const float* out_scale, char* err, size_t err_len);
 int mxmlp_get_params(mxmlp* h, float* params, char* err, size_t err_len);
 int mxmlp_set_params(mxmlp* h, const float* params, char* err, size_t err_len);
-/* y (n x outputs, physical units) for x (n x inputs). */
+/* y (n x outputs, physical units) for x (n x inputs). With the fused forward (mxmlp_set_fused) several
+ * host threads may call it on one network at the same time, while no call changes the network; every
+ * other use of a network is one call at a time. */
 int mxmlp_predict(mxmlp* h, const float* x, int64_t n, float* y, char* err, size_t err_len);
 /* The mean squared error of the normalised outputs over one batch and its gradient (grads may be
  * NULL), in parameter order. */
