@@ -976,7 +976,7 @@ class Net {
 
   // Forward of n samples (host arrays, n x inputs -> n x outputs, physical units).
   void predict(const float* x, long long n, float* y) {
-    const long long chunk = std::min(n, kChunk);
+    const long long chunk = std::min(n, fused_inference() ? kChunk : kLayeredChunk);
     Staging staging(*this, chunk);
     const Buf<float>&xd = staging.x(), &yd = staging.t();
     for (long long at = 0; at < n; at += chunk) {
@@ -999,7 +999,7 @@ class Net {
     check(hipMemcpyAsync(td.get(), t, std::size_t(n) * d_out_ * sizeof(float), hipMemcpyHostToDevice, s_), "hipMemcpy");
     ensure_loss();
     check(hipMemsetAsync(loss_sum_.get(), 0, sizeof(double), s_), "hipMemsetAsync");
-    if (fused_training()) {
+    if (fused_width()) {
       train_batch<false>(xd.get(), td.get(), n, nullptr);
       k_sum_parts<<<cdiv(np_, 256), 256, 0, s_>>>(part_.get(), np_, splits_of(n), order_.get(), grads_.get());
       check(hipGetLastError(), "k_sum_parts");
@@ -1027,7 +1027,7 @@ class Net {
     ensure(n);
     ensure_loss();
     check(hipMemsetAsync(loss_sum_.get(), 0, sizeof(double), s_), "hipMemsetAsync");
-    if (fused_training()) {
+    if (fused_width()) {
       TraceTable tr{};
       for (std::size_t q = 0; q < std::size_t(nl); ++q) {
         tr.h[q] = acts_[q].get();
@@ -1069,7 +1069,7 @@ class Net {
   float train(int epochs, int batch, float lr, uint64_t seed, double* seconds) {
     if (n_data_ < batch || batch < 64) throw std::invalid_argument("mlp: batch >= 64 and <= the data");
     const long long nb = n_data_ / batch;
-    const bool fused = fused_training();
+    const bool fused = fused_width();
     Buf<float> bx(fused ? 0 : std::size_t(batch) * d_in_), bt(fused ? 0 : std::size_t(batch) * d_out_);
     const Buf<long long>& idx = idx_;
     std::vector<long long> order(static_cast<std::size_t>(n_data_));
@@ -1156,7 +1156,7 @@ class Net {
   // layer-by-layer products; the same bits either way.
   void infer(const float* x, int n, float* y) {
     const int h = w_[1];
-    if (fused_ && h <= 256 && w_.size() - 1 <= std::size_t(kMaxLayers)) {
+    if (fused_inference()) {
       LayerTable L{};
       L.nl = layers();
       for (int l = 0; l < L.nl; ++l) {
@@ -1209,8 +1209,10 @@ class Net {
  private:
   static constexpr int kInPad = 32, kOutPad = 16;
 
-  // Samples predict takes to the device at a time.
-  static constexpr long long kChunk = 1 << 18;
+  // Samples predict takes to the device at a time: with the fused forward, which needs no memory beside
+  // the samples, and layer by layer, which holds every layer's activations, pre-activations and room
+  // for their gradients (8 bytes of each width per sample, kept: 8.6 GB for 16 layers of 1024).
+  static constexpr long long kChunk = 1 << 18, kLayeredChunk = 1 << 16;
 
   // A call's device copies of n host samples: their inputs, and their targets or outputs. The call
   // has them to itself: another one at the same time (mxmlp_predict may be called from several host
@@ -1244,6 +1246,11 @@ class Net {
     Buf<float> x_, t_;
   };
 
+  // The fused kernels, of inference and of training, are built for these widths; wider networks run and
+  // train layer by layer.
+  bool fused_width() const { return w_[1] <= 256 && layers() <= kMaxLayers; }
+  bool fused_inference() const { return fused_ && fused_width(); }
+
   void refresh_bf16() {
     k_to_bf16<<<cdiv(np_, 256), 256, 0, s_>>>(params_.get(), np_, copies());
     check(hipGetLastError(), "k_to_bf16");
@@ -1267,9 +1274,6 @@ class Net {
   void ensure_loss() {
     if (loss_sum_.size() == 0) loss_sum_ = Buf<double>(1);
   }
-
-  // The fused training step's kernels are built for these widths; wider networks train layer by layer.
-  bool fused_training() const { return w_[1] <= 256 && layers() <= kMaxLayers; }
 
   // Up to this many samples a workgroup takes one row tile.
   static constexpr int kOneRowTile = 8192;

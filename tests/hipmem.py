@@ -31,6 +31,14 @@ def check(rc: int, what: str) -> None:
         raise RuntimeError(f"{what}: HIP error {rc}")
 
 
+def free_bytes() -> int:
+    """Device memory not allocated."""
+    hip = _hip()
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    check(hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)), "hipMemGetInfo")
+    return free.value
+
+
 class DeviceArray:
     """n FP64 values in device memory."""
 

@@ -1,4 +1,5 @@
-"""The warm-start network's calls beside each other: predictions from several host threads at once."""
+"""The warm-start network's calls beside each other: predictions from several host threads at
+once, and what a prediction of many samples keeps on the device."""
 
 from __future__ import annotations
 
@@ -8,6 +9,7 @@ import numpy as np
 import pytest
 
 from autan_amd.mlp import MLP
+from hipmem import free_bytes
 
 pytestmark = pytest.mark.gpu
 
@@ -35,4 +37,22 @@ def test_predictions_from_several_threads():
     for t in threads:
         t.join()
     assert not wrong
+    m.close()
+
+
+@pytest.mark.parametrize("hidden,fused", [(320, True), (256, False)])
+def test_layered_prediction_holds_a_chunk_of_activations(hidden, fused):
+    """Layer by layer a prediction of many samples goes by chunks of 2^16, whose activations (BF16),
+    pre-activations (FP32) and gradients' room (BF16) of every layer stay on the device: 8 bytes per
+    value of a layer."""
+    m = MLP(7, hidden, 3, 5, seed=4)
+    m.set_fused(fused)
+    x = samples((1 << 18) + 3, 8)
+    m.predict(x[:64])
+    before = free_bytes()
+    y = m.predict(x)
+    grown = before - free_bytes()
+    held = (1 << 16) * (8 * sum(m.widths()[1:]) + 2 * 32)
+    assert grown <= held + (64 << 20)  # the chunk's samples and the allocator's granularity
+    np.testing.assert_array_equal(m.predict(x[-5000:]), y[-5000:])
     m.close()
