@@ -56,3 +56,12 @@ def test_layered_prediction_holds_a_chunk_of_activations(hidden, fused):
     assert grown <= held + (64 << 20)  # the chunk's samples and the allocator's granularity
     np.testing.assert_array_equal(m.predict(x[-5000:]), y[-5000:])
     m.close()
+
+
+def test_a_wide_network_holds_no_operand_packs():
+    """Networks wider than the fused kernels hold, per parameter, the FP32 weight, gradient and Adam's
+    two moments, the BF16 weight and a mask byte: nothing laid out for kernels that they never run."""
+    before = free_bytes()
+    m = MLP(7, 2048, 4, 5, seed=4)
+    assert before - free_bytes() <= m.param_count * (4 * 4 + 2 + 1) + (32 << 20)
+    m.close()
