@@ -1284,9 +1284,13 @@ class Net {
   static int tiles_of(int n) { return cdiv(n, kPackTile); }
   // Partial gradients of a batch: eight sample tiles each where that gives at most 8, one per XCD (at 56
   // tiles of weights for four hidden layers of 256, 4096 samples then make 448 workgroups; 16 take the
-  // same 11 us and cost k_adam 1 more).
+  // same 11 us and cost k_adam 1 more). From 4608 samples on, one per 512 samples up to 32, so that no
+  // FP32 chain gets longer than the layer-by-layer step's: with 8 a weight gradient's error against 64
+  // bits was 2.4e-7 of it at 131072 samples and 6e-7 at 524288, now 1.1e-7 and 1.5e-7, as there; and a
+  // narrow network, of few tiles of weights, has more workgroups (128-wide, three layers: 347 us a batch
+  // of 65536 with 8, 289 now; four layers of 256 at 8192: 86 and 87 us).
   static int splits_of(int n) {
-    const int tiles = tiles_of(n), want = std::max(1, std::min(8, cdiv(tiles, 8)));
+    const int tiles = tiles_of(n), want = std::max(std::min(8, cdiv(tiles, 8)), std::min(32, tiles / 16));
     return cdiv(tiles, cdiv(tiles, want));
   }
 

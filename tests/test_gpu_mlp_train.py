@@ -69,3 +69,26 @@ def test_an_epoch_is_its_batches(hidden):
     assert moved > 0 and np.abs(pa - p0).max() <= 1.01 * steps * lr
     assert np.linalg.norm(pa - pb) <= 2e-2 * moved
     assert loss == pytest.approx(last, rel=1e-3)
+
+
+def test_a_large_batch_keeps_its_gradients_chains_short():
+    """The weight gradients of 2^19 samples whose targets are noise, against FP64 sums of the traced dZ
+    and H: FP32 chains of c = 512 matrix products of 32 samples, then 32 partial sums. A chain of c
+    zero-mean terms grows as the square root of its length and each addition rounds its value by 0.42
+    2^-24 of it (the root mean square over a mantissa), so the chain ends 0.42 2^-24 sqrt(c / 2) of its
+    value off, and the sum of 32 such adds 0.42 2^-24 sqrt(32 / 2): 4.2e-7 in all; eight partial sums
+    would make it 8.1e-7."""
+    n, u = 1 << 19, 0.424 * 2.0**-24
+    x, _ = data(n, 7, 5, 3)
+    t = np.random.default_rng(4).standard_normal((n, 5)).astype(np.float32)
+    m = MLP(7, 64, 2, 5, seed=1)
+    _, g = m.gradients(x, t)
+    at = 0
+    w = m.widths()
+    for l in range(len(w) - 1):
+        h, dz = m.trace(x, t, "input", l).astype(np.float64), m.trace(x, t, "dz", l).astype(np.float64)
+        want = dz.T @ h
+        got = g[at : at + want.size].reshape(want.shape)
+        at += want.size + w[l + 1]
+        assert np.linalg.norm(got - want) <= u * np.hypot(np.sqrt(512 / 2), np.sqrt(32 / 2)) * np.linalg.norm(want), l
+    m.close()
