@@ -34,7 +34,9 @@ constexpr int kTileM = 64, kTileN = 64, kTileK = 32;
 constexpr int kPad = 8;  // LDS row padding (bf16) against bank conflicts
 
 inline void check(hipError_t e, const char* what) {
-  if (e != hipSuccess) throw std::runtime_error(std::string("E1101: ") + what + ": " + hipGetErrorString(e));
+  if (e == hipSuccess) return;
+  (void)hipGetLastError();  // reported here: the next launch's check must not find it
+  throw std::runtime_error(std::string("E1101: ") + what + ": " + hipGetErrorString(e));
 }
 
 // SiLU and its derivative through the logistic s(z) = 1 / (1 + e^-z), with the hardware exponential
@@ -1058,7 +1060,11 @@ class Net {
 
   // Training data resident on the device; epochs of shuffled batches with Adam.
   void set_data(const float* x, const float* t, long long n) {
-    if (data_x_.size() != std::size_t(n) * d_in_) {
+    // Without data until all of it is there: after a failed allocation train() refuses, and the next
+    // call makes every buffer again.
+    const bool as_many = n == n_data_;
+    n_data_ = 0;
+    if (!as_many) {
       data_x_ = Buf<float>(std::size_t(n) * d_in_);
       data_t_ = Buf<float>(std::size_t(n) * d_out_);
       idx_ = Buf<long long>(std::size_t(n));

@@ -1,8 +1,9 @@
 """The warm-start network's calls beside each other: predictions from several host threads at
-once, and what a prediction of many samples keeps on the device."""
+once, what calls keep on the device, and data that does not fit there."""
 
 from __future__ import annotations
 
+import ctypes
 import threading
 
 import numpy as np
@@ -64,4 +65,21 @@ def test_a_wide_network_holds_no_operand_packs():
     before = free_bytes()
     m = MLP(7, 2048, 4, 5, seed=4)
     assert before - free_bytes() <= m.param_count * (4 * 4 + 2 + 1) + (32 << 20)
+    m.close()
+
+
+def test_data_that_does_not_fit_leaves_none():
+    """Training data whose inputs fit the device (34 GB) and whose targets do not (550 GB): the call is
+    refused before it reads a sample, and training is until there is data again."""
+    m = MLP(1, 64, 1, 16, seed=1)
+    x, t = samples(64, 1)[:, :1].copy(), np.zeros((64, 16), np.float32)
+    loss, _ = m.train(x, t, epochs=1, batch=64, lr=0.0)
+    with pytest.raises(RuntimeError, match="hipMalloc"):
+        m._call(m.lib.mxmlp_set_data, ctypes.c_void_p(x.ctypes.data), ctypes.c_void_p(t.ctypes.data),
+                ctypes.c_int64(1 << 33))
+    out, sec = ctypes.c_float(), ctypes.c_double()
+    with pytest.raises(RuntimeError, match="batch >= 64 and <= the data"):
+        m._call(m.lib.mxmlp_train, ctypes.c_int32(1), ctypes.c_int32(64), ctypes.c_float(0.0), ctypes.c_uint64(0),
+                ctypes.byref(out), ctypes.byref(sec))
+    assert m.train(x, t, epochs=1, batch=64, lr=0.0)[0] == pytest.approx(loss, rel=1e-6)
     m.close()
