@@ -366,14 +366,18 @@ __global__ __launch_bounds__(kBlock) void k_grad(Dev<C> d) {
 // records), then every stencil entry gathers its primitives from LDS through a 16-bit position.
 // Weights, positions and the limiter's face offsets stream in the wave-sliced layout. The sums,
 // bounds and minima run in the same order as k_grad.
-// OCC > 0 asks the compiler for OCC waves per SIMD (registers capped accordingly): a variant for
-// the autotuner, same bits.
 // Bound by the stencil stream's bytes on a large mesh and by the loads' latency on a small one: kAhead
 // entries (and as many of the limiter's offsets) are in flight while the ones before are summed, the
 // first of them before the table is staged. With one entry ahead and nothing before the table: 308 us
 // on a 2.3M-cell channel in fp32 (1.25 GB; 270 now, 4.6 TB/s), 37 us on 33k cells (26), 57 us on 172k in
 // fp64 (50). Two entries ahead in fp64, whose four would cost a wave per SIMD (1.11 against 1.15 ms for
-// three steps of 172k cells); in fp32 two, four and six take the same time on large meshes.
+// three steps of 172k cells); in fp32 two, four and six take the same time on large meshes, four at 98
+// registers and four waves per SIMD (75 and six with one).
+// OCC > 0 asks the compiler for OCC waves per SIMD (72 registers at 7, 64 at 8): variants for the
+// autotuner, same bits. They hold one entry ahead and nothing over the table, as more would be spilled
+// (55 registers at 7 with four: 1889 us a step of a 1.2M-cell channel in fp32, 974 without; 930 with OCC
+// 0); in fp64, which spills all the same, up to the lane's own entries with a branch (7 registers fewer:
+// 1106 and 1144 us on 384k tetrahedra), in fp32 the slice's (1205 and 1333 us at 8).
 // A load of data read once per launch: with NT, marked non-temporal (streamed past the caches'
 // replacement, leaving them to the data other blocks read again); the same value either way.
 template <bool NT, class T>
@@ -387,7 +391,9 @@ __device__ __forceinline__ T stream_load(const T* p) {
 
 template <class C, bool LIMITER, int OCC = 0, bool NT = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 ? OCC : 1))) void k_grad_lds(Dev<C> d) {
-  constexpr int kAhead = std::is_same_v<C, float> ? 4 : 2;
+  constexpr bool kEarly = OCC == 0;
+  constexpr int kAhead = !kEarly ? 1 : std::is_same_v<C, float> ? 4 : 2;
+  constexpr bool kSlice = kEarly || std::is_same_v<C, float>;
   extern __shared__ __align__(16) unsigned char smem[];
   C* tab = reinterpret_cast<C*>(smem);
   const int blk = cell_block(d);
@@ -405,7 +411,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
   const int slice = __builtin_amdgcn_readfirstlane(c) / kWave, lane = threadIdx.x % kWave;
   const bool any = __builtin_amdgcn_readfirstlane(c) < d.nc;
   const long long s0 = any ? d.soff[slice] : 0;
-  const int longest = any ? static_cast<int>((d.soff[slice + 1] - s0) / kWave) : 0;
+  const int longest = !kSlice ? len : any ? static_cast<int>((d.soff[slice + 1] - s0) / kWave) : 0;
   // The entries' positions and weights, kAhead of them in flight while the ones before are summed
   // (the first before the table is staged); the sums run in entry order.
   int l_next[kAhead];
@@ -420,8 +426,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
       w_next[u][2] = stream_load<NT>(d.sw2 + k);
     }
   };
-  if (longest > 0) entries(0);
-  const W5<C> wc = inside ? load_w(d.prim, c) : W5<C>{};
+  if (kEarly && longest > 0) entries(0);
+  W5<C> wc{};
+  if (kEarly && inside) wc = load_w(d.prim, c);
   for (int j = threadIdx.x; j < tn; j += kBlock) {
     const int e = d.tent[t0 + j];
     const W5<C> w = e >= 0 ? load_w(d.prim, e) : load_w(d.prim_b, -e - 1);
@@ -433,6 +440,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
   }
   __syncthreads();
   if (!inside) return;
+  if constexpr (!kEarly) {
+    wc = load_w(d.prim, c);
+    if (longest > 0) entries(0);
+  }
   const C wcv[5] = {wc.r, wc.u, wc.v, wc.w, wc.p};
   double acc[15];
 #pragma unroll
@@ -474,7 +485,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
   if constexpr (LIMITER) {
     C r_next[kAhead][3];
     const long long i0 = d.ioff[slice];
-    const int ilongest = static_cast<int>((d.ioff[slice + 1] - i0) / kWave);
+    const int ilongest = !kSlice ? ilen : static_cast<int>((d.ioff[slice + 1] - i0) / kWave);
     auto offsets = [&](int j0) {
 #pragma unroll
       for (int u = 0; u < kAhead; ++u) {
