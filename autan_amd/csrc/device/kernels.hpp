@@ -622,8 +622,9 @@ struct StagedCells {
 // Whether a face's warp term with zero moments is zero in every component: its directions are zeros
 // then (gradient times zero), and so are their products with the mean state, unless one of the
 // factors is infinite or not a number, which this finds in the two sides' gradients and limiters, the
-// mean state, its |v|^2 and its enthalpy density (which bounds its momentum). Adding such a zero to a
-// flux could only turn -0 into +0, which no sum of fluxes from +0 shows. 98.5 % of a channel's faces
+// mean state, its |v|^2 and its enthalpy density. (Not the momentum rho v_i: the mean's density is at most
+// half the largest number, so it is finite for |v_i| <= 2, and beyond at most the enthalpy density's
+// rho |v|^2 / 2; nor sums of gradients: each is multiplied by its zero first.) Adding such a zero to a flux could only turn -0 into +0, which no sum of fluxes from +0 shows. 98.5 % of a channel's faces
 // are flat: 47 multiply-adds instead of the term's 370 instructions, a third of the interior face's
 // arithmetic (172k cells in fp64: faces_rk 49.0 us before, 46.8 now; 2.3M in fp32: faces_first_rk 354 and
 // 340, faces_rk unchanged, bound by its gathers).
