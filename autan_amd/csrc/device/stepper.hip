@@ -1064,10 +1064,17 @@ class Stepper final : public StepperBase {
     }
     if (n == 0) return;
     if (n > INT32_MAX / 3) throw std::invalid_argument("face_force: too many faces");
-    // The staging stays with the stepper, as large as its longest list (at most its boundary).
-    if (force_list_.size() < static_cast<std::size_t>(n)) {
-      force_list_ = Buffer<int>(static_cast<std::size_t>(n));
-      force_out_ = Buffer<double>(3 * static_cast<std::size_t>(n));
+    const std::size_t count = static_cast<std::size_t>(n), kept = static_cast<std::size_t>(nb_);
+    if (count > kept) {  // faces listed more than once: staging of its own
+      Buffer<int> list(count);
+      Buffer<double> out(3 * count);
+      face_force_into(faces, n, force, list.get(), out.get());
+      return;
+    }
+    // Staging for every boundary face stays with the stepper; there once its second part is.
+    if (force_out_.size() == 0) {
+      force_list_ = Buffer<int>(kept);
+      force_out_ = Buffer<double>(3 * kept);
     }
     face_force_into(faces, n, force, force_list_.get(), force_out_.get());
   }

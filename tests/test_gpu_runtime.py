@@ -45,6 +45,19 @@ def test_face_force_matches_oracle_bit_for_bit(name, policy):
     np.testing.assert_array_equal(dev.face_force(faces[::3]), ora.face_force(u1, faces[::3]))
 
 
+def test_face_force_of_faces_listed_more_than_once():
+    """Lists longer than the boundary take staging of their own, between lists that use the kept one."""
+    case = cases.tets_case(3)
+    with DeviceStepper(case.mesh, case.scheme, "fp64", case.bc_kind, case.bc, case.source) as dev:
+        dev.upload(case.u)
+        faces = np.arange(case.mesh.n_interior, case.mesh.n_faces, dtype=np.int32)
+        few = dev.face_force(faces[:7])
+        many = dev.face_force(np.tile(faces, 5))
+        once = dev.face_force(faces)
+        np.testing.assert_array_equal(many, np.tile(once, (1, 5)))
+        np.testing.assert_array_equal(few, once[:, :7])
+
+
 @pytest.mark.parametrize("policy", ["fp64", "fp32+acc64"])
 def test_loads_are_exact_sums_of_the_face_forces(policy):
     case = cases.bump_case(16, 12, 8, hybrid=True)
