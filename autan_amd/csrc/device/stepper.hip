@@ -974,7 +974,12 @@ class Stepper final : public StepperBase {
       graph_step(cfl, true);
     } else {
       bstate_fresh_ = true;  // of the first residual alone (a graph's is recorded for any step)
-      enqueue_step(cfl, false, 0.0, true);
+      try {
+        enqueue_step(cfl, false, 0.0, true);
+      } catch (...) {
+        bstate_fresh_ = false;  // a launch before it failed
+        throw;
+      }
     }
     finish(residuals, invalid);
     eval_norms(reported);
