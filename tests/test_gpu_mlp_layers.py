@@ -74,7 +74,7 @@ def split(params, w):
     return mo.unpack(params, w)
 
 
-@pytest.mark.parametrize("n", [200, 1024])
+@pytest.mark.parametrize("n", [200, 1024, 8205])
 def test_forward_layers_within_their_rounding(n):
     m = trained(1)
     x, t = data(n, 3)
@@ -103,7 +103,7 @@ def test_forward_layers_within_their_rounding(n):
     np.testing.assert_array_equal(y, zl * norm[3] + norm[2])
 
 
-@pytest.mark.parametrize("n", [200, 1024])
+@pytest.mark.parametrize("n", [200, 1024, 8205])
 def test_backward_layers_within_their_rounding(n):
     m = trained(2)
     x, t = data(n, 5)

@@ -3,8 +3,8 @@ layer's gradients) where its tiles can go wrong: batches around the 16- and 32-s
 the switch between one and two row tiles per workgroup, every width it is built for and the layered
 path past them, one hidden layer and many, inputs and outputs that fill their padding; against the FP64
 oracle of the BF16 network, whose gradients the kernels' own roundings of the activations and of dZ
-leave within the bound below. And an epoch on whole batches against the same batches given one by one
-to gradients() and adam_step()."""
+leave within the bound below. And epochs of one batch and of batches that are alike against the same
+batches given one by one to gradients() and adam_step(), and which samples an epoch's batches take."""
 
 from __future__ import annotations
 
@@ -91,4 +91,94 @@ def test_a_large_batch_keeps_its_gradients_chains_short():
         got = g[at : at + want.size].reshape(want.shape)
         at += want.size + w[l + 1]
         assert np.linalg.norm(got - want) <= u * np.hypot(np.sqrt(512 / 2), np.sqrt(32 / 2)) * np.linalg.norm(want), l
+    m.close()
+
+
+def pair(hidden, x, t):
+    a, b = MLP(7, hidden, 3, 5, seed=2), MLP(7, hidden, 3, 5, seed=2)
+    for m in (a, b):
+        m.fit_normalization(x, t)
+    return a, b
+
+
+@pytest.mark.parametrize("hidden,n", [(128, 500), (192, 500), (64, 8200), (128, 8193), (192, 8223), (256, 8200)])
+def test_an_epoch_of_one_batch_at_every_width_and_tile(hidden, n):
+    """As test_an_epoch_is_its_batches, to its bounds, at the other widths and past one row tile per
+    workgroup."""
+    steps, lr = 3, 1e-3
+    x, t = data(n, 7, 5, 3)
+    a, b = pair(hidden, x, t)
+    p0 = a.params()
+    loss, _ = a.train(x, t, epochs=steps, batch=n, lr=lr, seed=1)
+    for _ in range(steps):
+        last, _ = b.gradients(x, t)
+        b.adam_step(lr)
+    moved = np.linalg.norm(b.params() - p0)
+    assert moved > 0 and np.linalg.norm(a.params() - b.params()) <= 2e-2 * moved
+    assert loss == pytest.approx(last, rel=1e-3)
+
+
+@pytest.mark.parametrize("hidden,batch", [(64, 100), (256, 256), (128, 8200)])
+def test_every_batch_of_an_epoch_is_its_own(hidden, batch):
+    """Four batches whose samples the shuffle chooses, at weights that stand still: the epoch's loss is
+    the mean over its samples, here the count of those with a large target, 37 in all and at most the
+    five samples left over fewer. A batch taken twice would make the count another, or by its size a
+    multiple of four under every seed. With as many samples as the batches take, the loss is gradients()'s."""
+    left, large = 5, 37
+    n = 4 * batch + left
+    x, _ = data(n, 7, 5, 3)
+    t = np.zeros((n, 5), np.float32)
+    t[np.random.default_rng(6).choice(n, large, replace=False)] = 1e4  # a large sample's squared error: 1e8, others' below 1
+    m = MLP(7, hidden, 3, 5, seed=2)
+    counts = []
+    for seed in range(6):
+        loss, _ = m.train(x, t, epochs=1, batch=batch, lr=0.0, seed=seed)
+        count = loss * 4 * batch / 1e8
+        assert abs(count - round(count)) <= 0.02 and large - left <= round(count) <= large, count
+        counts.append(round(count))
+    assert any(c % 4 for c in counts)
+    whole = 4 * batch
+    t[:, 0] += np.arange(n) ** 2  # targets unlike each other
+    want, _ = m.gradients(x[:whole], t[:whole])
+    loss, _ = m.train(x[:whole], t[:whole], epochs=1, batch=batch, lr=0.0, seed=7)
+    # FP32 squared errors, summed to 64 lanes in FP32 and further in FP64, in another order
+    assert loss == pytest.approx(want, rel=1e-5)
+    m.close()
+
+
+def test_steps_within_an_epoch_are_counted():
+    """Batches all alike: an epoch of four is four of gradients() and adam_step(), whose bias corrections
+    depend on the count."""
+    one, lr = 128, 1e-3
+    x, t = data(1, 7, 5, 3)
+    x, t = np.tile(x, (4 * one, 1)), np.tile(t, (4 * one, 1))
+    a, b = MLP(7, 128, 3, 5, seed=2), MLP(7, 128, 3, 5, seed=2)
+    p0 = a.params()
+    a.train(x, t, epochs=1, batch=one, lr=lr, seed=1)
+    for _ in range(4):
+        b.gradients(x[:one], t[:one])
+        b.adam_step(lr)
+    moved = np.linalg.norm(b.params() - p0)
+    assert moved > 0 and np.linalg.norm(a.params() - b.params()) <= 1e-5 * moved
+
+
+@pytest.mark.parametrize("hidden,layers", [(64, 2), (192, 3), (256, 2)])
+@pytest.mark.parametrize("n", [17, 33, 8191, 8193, 8209])
+def test_the_last_tile_alone(hidden, layers, n):
+    """Targets of the last tile of 32 that are so large that its samples, one of 8193, are the gradient:
+    a tile dropped, read twice or masked wrongly is all of it. To the bound of the tiles' edges test."""
+    x, t = data(n, 7, 5, n)
+    t[(n - 1) // 32 * 32 :] += 1e6
+    m = MLP(7, hidden, layers, 5, seed=n)
+    norm = [np.asarray(a, np.float64) for a in m.norm]
+    loss, g = m.gradients(x, t)
+    l_o, g_o = mo.loss_and_gradients(m.params(), m.widths(), x, t, norm, 5, bf=True)
+    assert abs(loss - l_o) <= 1e-2 * l_o
+    at = 0
+    w = m.widths()
+    for l in range(len(w) - 1):
+        for size in (w[l + 1] * w[l], w[l + 1]):
+            seg = slice(at, at + size)
+            at += size
+            assert np.linalg.norm(g[seg] - g_o[seg]) <= 5e-2 * np.linalg.norm(g_o[seg]), (l, size)
     m.close()

@@ -3,6 +3,7 @@ each through the C ABI against the oracle (or a closed form) on the same inputs.
 
 from __future__ import annotations
 
+import ctypes
 import math
 
 import numpy as np
@@ -225,3 +226,34 @@ def test_a_residual_between_evaluation_and_solve_is_the_host_calls(policy):
             np.testing.assert_array_equal(states[1], states[0])
         finally:
             a.free()
+
+
+@pytest.mark.parametrize("kind", ["pinned", "managed", "misaligned"])
+def test_a_residual_of_memory_the_kernels_leave_alone(kind):
+    """Pinned host memory, managed memory and an address that is no multiple of 8 go through copies, in
+    and out: the host call's bits."""
+    from hipmem import _D2H, _H2D, _hip, check
+
+    case = cases.tets_case(3)
+    n5 = 5 * case.mesh.n_cells
+    hip = _hip()
+    u, out = np.ascontiguousarray(case.u, dtype=np.float64).reshape(-1), np.empty(n5)
+    with DeviceStepper(case.mesh, case.scheme, "fp64", case.bc_kind, case.bc, case.source) as dev:
+        want = dev.residual(case.u).reshape(-1)
+        p = ctypes.c_void_p()
+        size, off = 8 * n5 + 8, 4 if kind == "misaligned" else 0
+        if kind == "pinned":
+            check(hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(size), 0), "hipHostMalloc")
+        elif kind == "managed":
+            check(hip.hipMallocManaged(ctypes.byref(p), ctypes.c_size_t(size), 1), "hipMallocManaged")
+        else:
+            check(hip.hipMalloc(ctypes.byref(p), size), "hipMalloc")
+        try:
+            for _ in range(2):
+                check(hip.hipMemcpy(p.value + off, u.ctypes.data, 8 * n5, _H2D), "hipMemcpy")
+                dev.residual_device(p.value + off, p.value + off)
+                check(hip.hipStreamSynchronize(None), "hipStreamSynchronize")
+                check(hip.hipMemcpy(out.ctypes.data, p.value + off, 8 * n5, _D2H), "hipMemcpy")
+                np.testing.assert_array_equal(out, want)
+        finally:
+            check((hip.hipHostFree if kind == "pinned" else hip.hipFree)(p), "free")
