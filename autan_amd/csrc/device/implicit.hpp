@@ -655,6 +655,23 @@ __device__ __forceinline__ void impl_tangent(const double* __restrict__ dwdu, co
   }
 }
 
+// Marks the listed cells and the cells of their gradient stencils: those whose tangents the boundary term
+// reads. Threads that mark one cell write the same byte.
+template <class C>
+__global__ __launch_bounds__(kBlock) void k_impl_near(Dev<C> d, const int* __restrict__ cells, int count,
+                                                      unsigned char* __restrict__ mark) {
+  const int t = blockIdx.x * kBlock + threadIdx.x;
+  if (t >= count) return;
+  const int c = cells[t];
+  mark[c] = 1;
+  const long long at = d.soff[c / kWave] + c % kWave;
+  const int len = d.slen[c];
+  for (int j = 0; j < len; ++j) {
+    const int e = d.sidx[at + static_cast<long long>(j) * kWave];
+    if (e >= 0) mark[e] = 1;
+  }
+}
+
 // The primitive tangent dW/dq v (impl_tangent) of the listed cells, 5 consecutive values per cell in the
 // compute type, for the boundary term's stencils.
 template <class C>

@@ -456,71 +456,74 @@ class Stepper final : public StepperBase {
       ++off[static_cast<std::size_t>(neighbour_host_[f]) + 1];
     }
     for (std::size_t c = 0; c < n; ++c) off[c + 1] += off[c];
-    std::vector<int2> ent(std::max<std::size_t>(2 * ni, 1));
+    std::vector<int> nbr(std::max<std::size_t>(2 * ni, 1));  // the other cell of each of a row's faces
     std::vector<int> fill(off.begin(), off.end() - 1);
     for (std::size_t f = 0; f < ni; ++f) {
       const int o = owner_host_[f], nb = neighbour_host_[f];
-      // Row owner: the upper block (index f), other cell the neighbour; row neighbour: the lower
-      // block (index ni + f), other cell the owner.
-      ent[static_cast<std::size_t>(fill[static_cast<std::size_t>(o)]++)] = make_int2(static_cast<int>(f), nb);
-      ent[static_cast<std::size_t>(fill[static_cast<std::size_t>(nb)]++)] = make_int2(static_cast<int>(ni + f), o);
+      nbr[static_cast<std::size_t>(fill[static_cast<std::size_t>(o)]++)] = nb;
+      nbr[static_cast<std::size_t>(fill[static_cast<std::size_t>(nb)]++)] = o;
     }
+    // Coloured in cell order; of two neighbours the lower colour has one above it.
     colour_host_.assign(n, -1);
-    int colours = 0;
-    std::vector<char> seen;
+    std::vector<char> above(n, 0);
+    std::vector<int> seen(1, -1);  // by colour, the last cell beside one of it; one more than the colours
     for (std::size_t c = 0; c < n; ++c) {
-      seen.assign(static_cast<std::size_t>(colours) + 1, 0);
       for (int k = off[c]; k < off[c + 1]; ++k) {
-        const int other = ent[static_cast<std::size_t>(k)].y;
-        if (colour_host_[static_cast<std::size_t>(other)] >= 0) seen[static_cast<std::size_t>(colour_host_[static_cast<std::size_t>(other)])] = 1;
+        const int q = colour_host_[static_cast<std::size_t>(nbr[static_cast<std::size_t>(k)])];
+        if (q >= 0) seen[static_cast<std::size_t>(q)] = static_cast<int>(c);
       }
-      int k = 0;
-      while (seen[static_cast<std::size_t>(k)] != 0) ++k;
-      colour_host_[c] = k;
-      colours = std::max(colours, k + 1);
+      int own = 0;
+      while (seen[static_cast<std::size_t>(own)] == static_cast<int>(c)) ++own;
+      if (static_cast<std::size_t>(own) + 1 == seen.size()) seen.push_back(-1);
+      colour_host_[c] = own;
+      for (int k = off[c]; k < off[c + 1]; ++k) {
+        const auto other = static_cast<std::size_t>(nbr[static_cast<std::size_t>(k)]);
+        const int q = colour_host_[other];
+        if (q >= 0 && q != own) above[q > own ? c : other] = 1;
+      }
     }
+    const int colours = static_cast<int>(seen.size()) - 1;
     // The rows by position (implicit.hpp): colour by colour, in each the cells with a neighbour of a
     // higher colour first (the way back down a sweep relaxes them alone, plan_relax), then the others;
     // in each of these groups ascending, but within every 80 slices ordered by their entries, so that
     // few slices pad rows of unlike lengths (2.6-9 % of the slots as they come, 0.2-0.7 % so).
-    std::vector<char> above(n, 0);
+    std::vector<int> group(n);
+    std::vector<int> size(2 * static_cast<std::size_t>(colours), 0);
     for (std::size_t c = 0; c < n; ++c) {
-      for (int k = off[c]; k < off[c + 1]; ++k) {
-        const int other = ent[static_cast<std::size_t>(k)].y;
-        if (colour_host_[static_cast<std::size_t>(other)] > colour_host_[c]) above[c] = 1;
-      }
+      group[c] = 2 * colour_host_[c] + (above[c] != 0 ? 0 : 1);
+      ++size[static_cast<std::size_t>(group[c])];
     }
-    std::vector<std::vector<int>> groups(2 * static_cast<std::size_t>(colours));
-    for (std::size_t c = 0; c < n; ++c) {
-      groups[2 * static_cast<std::size_t>(colour_host_[c]) + (above[c] ? 0 : 1)].push_back(static_cast<int>(c));
-    }
-    std::vector<int> cells, slot{0};
+    std::vector<int> begin(size.size());
     colour_off_.assign(1, 0);
     colour_above_.clear();
-    auto entries = [&](int c) { return c < 0 ? 0 : off[static_cast<std::size_t>(c) + 1] - off[static_cast<std::size_t>(c)]; };
-    for (std::size_t g = 0; g < groups.size(); ++g) {
-      auto& rows = groups[g];
-      constexpr std::size_t kWindow = 80 * kSlice;
-      for (std::size_t w = 0; w < rows.size(); w += kWindow) {
-        std::stable_sort(rows.begin() + static_cast<std::ptrdiff_t>(w),
-                         rows.begin() + static_cast<std::ptrdiff_t>(std::min(rows.size(), w + kWindow)),
-                         [&](int a, int b) { return entries(a) < entries(b); });
-      }
-      rows.resize((rows.size() + kSlice - 1) / kSlice * kSlice, -1);
-      for (std::size_t p = 0; p < rows.size(); p += kSlice) {
-        int longest = 0;
-        for (std::size_t i = p; i < p + kSlice; ++i) longest = std::max(longest, entries(rows[i]));
-        slot.push_back(slot.back() + longest);
-      }
-      cells.insert(cells.end(), rows.begin(), rows.end());
-      const int end = static_cast<int>(cells.size() / kSlice);
+    int end = 0;  // in slices
+    for (std::size_t g = 0; g < size.size(); ++g) {
+      begin[g] = kSlice * end;
+      end += (size[g] + kSlice - 1) / kSlice;
       if (g % 2 == 0) {
         colour_above_.push_back(end - colour_off_.back());
       } else {
         colour_off_.push_back(end);
       }
     }
-    groups.clear();
+    std::vector<int> cells(static_cast<std::size_t>(end) * kSlice, -1);
+    std::vector<int> at(begin);
+    for (std::size_t c = 0; c < n; ++c) {
+      cells[static_cast<std::size_t>(at[static_cast<std::size_t>(group[c])]++)] = static_cast<int>(c);
+    }
+    auto entries = [&](int c) { return c < 0 ? 0 : off[static_cast<std::size_t>(c) + 1] - off[static_cast<std::size_t>(c)]; };
+    constexpr int kWindow = 80 * kSlice;
+    for (std::size_t g = 0; g < size.size(); ++g) {
+      for (int w = 0; w < size[g]; w += kWindow) {
+        order_rows(cells.data() + begin[g] + w, std::min(size[g] - w, kWindow), entries);
+      }
+    }
+    std::vector<int> slot(static_cast<std::size_t>(end) + 1, 0);
+    for (int q = 0; q < end; ++q) {
+      int longest = 0;
+      for (int i = kSlice * q; i < kSlice * (q + 1); ++i) longest = std::max(longest, entries(cells[static_cast<std::size_t>(i)]));
+      slot[static_cast<std::size_t>(q) + 1] = slot[static_cast<std::size_t>(q)] + longest;
+    }
     slices_ = colour_off_.back();
     std::vector<int> bo;
     for (std::size_t c = 0; c < n; ++c) {
@@ -534,7 +537,7 @@ class Stepper final : public StepperBase {
     nbo_ = static_cast<int>(bo.size());
     if (nbo_ > 0) bocells_.upload(bo, stream_);
     // The cells whose tangents the boundary term reads: those and their stencils'.
-    if (nbo_ > 0) near_.upload(stencil_cells(bo), stream_);
+    if (nbo_ > 0) near_.upload(stencil_cells(), stream_);
     // Each interior face's entries in its two rows (slot times kSlice plus the row's place in its
     // slice), a row's entries in ascending face order, and the other cell's position of each.
     std::vector<int> rank(n);
@@ -545,16 +548,16 @@ class Stepper final : public StepperBase {
     if (slots * kSlice > std::size_t(std::numeric_limits<int>::max())) throw std::invalid_argument("implicit step: too many faces");
     std::vector<int> other(std::max<std::size_t>(slots * kSlice, 1), -1);
     std::vector<int2> face_at(std::max<std::size_t>(ni, 1));
-    std::vector<int> pfill(n, 0);
-    auto next_entry = [&](int c) {
-      const int p = rank[static_cast<std::size_t>(c)];
-      return kSlice * (slot[static_cast<std::size_t>(p / kSlice)] + pfill[static_cast<std::size_t>(c)]++) + p % kSlice;
-    };
+    std::vector<int> next(n);  // each row's next entry
+    for (std::size_t c = 0; c < n; ++c) next[c] = kSlice * slot[static_cast<std::size_t>(rank[c] / kSlice)] + rank[c] % kSlice;
     for (std::size_t f = 0; f < ni; ++f) {
-      const int o = owner_host_[f], nb = neighbour_host_[f];
-      const int ko = next_entry(o), kn = next_entry(nb);
-      other[static_cast<std::size_t>(ko)] = rank[static_cast<std::size_t>(nb)];
-      other[static_cast<std::size_t>(kn)] = rank[static_cast<std::size_t>(o)];
+      const auto o = static_cast<std::size_t>(owner_host_[f]), nb = static_cast<std::size_t>(neighbour_host_[f]);
+      const int ko = next[o];
+      next[o] += kSlice;
+      const int kn = next[nb];
+      next[nb] += kSlice;
+      other[static_cast<std::size_t>(ko)] = rank[nb];
+      other[static_cast<std::size_t>(kn)] = rank[o];
       face_at[f] = make_int2(ko, kn);
     }
     rslot_.upload(slot, stream_);
@@ -589,24 +592,47 @@ class Stepper final : public StepperBase {
     implicit_ready_ = true;
   }
 
-  // The listed cells and the cells of their gradient stencils, ascending (from the device's stencil).
-  std::vector<int> stencil_cells(const std::vector<int>& list) {
-    std::vector<long long> soff(soff_.size());
-    std::vector<int> slen(slen_.size()), sidx(sidx_.size());
-    soff_.download(soff.data(), soff.size(), stream_);
-    slen_.download(slen.data(), slen.size(), stream_);
-    sidx_.download(sidx.data(), sidx.size(), stream_);
-    check(hipStreamSynchronize(stream_), "implicit_setup");
-    std::vector<int> out(list);
-    for (const int c : list) {
-      const long long base = soff[static_cast<std::size_t>(c / kWave)] + c % kWave;
-      for (int j = 0; j < slen[static_cast<std::size_t>(c)]; ++j) {
-        const int e = sidx[static_cast<std::size_t>(base + static_cast<long long>(j) * kWave)];
-        if (e >= 0) out.push_back(e);
-      }
+  // At most a window's rows ordered by their entries, rows with as many in the order they have: counted
+  // where the lengths differ by few (sorting took half of a first call's set-up).
+  template <class Entries>
+  static void order_rows(int* rows, int count, const Entries& entries) {
+    constexpr int kLengths = 64;
+    int least = INT32_MAX, most = 0;
+    bool ordered = true;
+    for (int i = 0; i < count; ++i) {
+      const int e = entries(rows[i]);
+      ordered = ordered && e >= most;
+      least = std::min(least, e);
+      most = std::max(most, e);
     }
-    std::sort(out.begin(), out.end());
-    out.erase(std::unique(out.begin(), out.end()), out.end());
+    if (ordered) return;
+    if (most - least >= kLengths) {
+      std::stable_sort(rows, rows + count, [&](int a, int b) { return entries(a) < entries(b); });
+      return;
+    }
+    std::array<int, kLengths + 1> at{};
+    for (int i = 0; i < count; ++i) ++at[static_cast<std::size_t>(entries(rows[i]) - least) + 1];
+    for (std::size_t k = 1; k < at.size(); ++k) at[k] += at[k - 1];
+    const std::vector<int> from(rows, rows + count);
+    for (const int c : from) rows[at[static_cast<std::size_t>(entries(c) - least)]++] = c;
+  }
+
+  // The cells with boundary faces (bocells_) and the cells of their gradient stencils, ascending: marked
+  // on the device, whose stencils are the only ones left (a byte per cell comes back; the stencils of a
+  // 7.9M-cell channel are 0.7 GB).
+  std::vector<int> stencil_cells() {
+    Buffer<unsigned char> mark(static_cast<std::size_t>(nc_));
+    check(hipMemsetAsync(mark.get(), 0, mark.size(), stream_), "hipMemsetAsync");
+    launch("impl_near", [&] {
+      k_impl_near<C><<<blocks(nbo_), kBlock, 0, stream_>>>(dev(), bocells_.get(), nbo_, mark.get());
+    });
+    std::vector<unsigned char> host(mark.size());
+    mark.download(host.data(), host.size(), stream_);
+    check(hipStreamSynchronize(stream_), "implicit_setup");
+    std::vector<int> out;
+    for (int c = 0; c < nc_; ++c) {
+      if (host[static_cast<std::size_t>(c)] != 0) out.push_back(c);
+    }
     return out;
   }
 
