@@ -1404,8 +1404,9 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
 // The step's reductions, one block per case: its exact-sum slots added into its words (integer
 // sums: any order gives the same words), and the least of its face blocks' time-step keys. One block,
 // so bound by the chain of its loads: each wave takes nslot / 16 slots and has all their words in
-// flight, then adds them into LDS. With one thread per word adding 64 slots in turn this took 17 us of
-// every step (28 on 786k cells), now 5.3.
+// flight, then adds them into LDS; the rest is the face blocks' keys, whose number grows with the mesh. With
+// one thread per word adding 64 slots in turn this took 17 us of a step of 33k cells, now 5.3; 28 of 796k
+// tetrahedra, now 8.8; 32 of a 2.3M-cell channel, now 10; 43 of 7.9M cells, now 15.7.
 __global__ __launch_bounds__(1024) void k_step_reduce(const long long* __restrict__ nslots, int nslot,
                                                       const unsigned long long* __restrict__ partial,
                                                       const int* __restrict__ fcbeg, const int* __restrict__ cflags,

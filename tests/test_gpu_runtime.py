@@ -257,3 +257,40 @@ def test_a_residual_of_memory_the_kernels_leave_alone(kind):
                 np.testing.assert_array_equal(out, want)
         finally:
             check((hip.hipHostFree if kind == "pinned" else hip.hipFree)(p), "free")
+
+
+@pytest.mark.parametrize("mode", [0, 1])  # hipStreamCaptureModeGlobal, ThreadLocal
+def test_a_captured_residual_replays(mode):
+    """residual_device recorded into a caller's graph: every replay reads the caller's state as it is
+    then, with the stepper's own work between the replays."""
+    from hipmem import DeviceArray, Stream, _hip, check
+
+    hip = _hip()
+    hip.hipStreamBeginCapture.argtypes = [ctypes.c_void_p, ctypes.c_int]
+    hip.hipStreamEndCapture.argtypes = [ctypes.c_void_p, ctypes.POINTER(ctypes.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [ctypes.POINTER(ctypes.c_void_p)] + 3 * [ctypes.c_void_p] + [ctypes.c_size_t]
+    hip.hipGraphLaunch.argtypes = 2 * [ctypes.c_void_p]
+    hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [ctypes.c_void_p]
+    case = cases.tets_case(5)
+    u, r, s = DeviceArray(5 * case.mesh.n_cells), DeviceArray(5 * case.mesh.n_cells), Stream()
+    graph, replay = ctypes.c_void_p(), ctypes.c_void_p()
+    with DeviceStepper(case.mesh, case.scheme, "fp64", case.bc_kind, case.bc, case.source) as dev:
+        u.copy_from(case.u)
+        dev.residual_device(u.ptr, r.ptr, s.handle)
+        s.synchronize()
+        check(hip.hipStreamBeginCapture(s.handle, mode), "hipStreamBeginCapture")
+        dev.residual_device(u.ptr, r.ptr, s.handle)
+        check(hip.hipStreamEndCapture(s.handle, ctypes.byref(graph)), "hipStreamEndCapture")
+        check(hip.hipGraphInstantiate(ctypes.byref(replay), graph, None, None, 0), "hipGraphInstantiate")
+        for k in range(3):
+            state = (1.0 + 0.01 * k) * case.u
+            want = dev.residual(state).reshape(-1)
+            u.copy_from(state)
+            check(hip.hipGraphLaunch(replay, s.handle), "hipGraphLaunch")
+            s.synchronize()
+            np.testing.assert_array_equal(r.numpy(), want)
+        check(hip.hipGraphExecDestroy(replay), "hipGraphExecDestroy")
+        check(hip.hipGraphDestroy(graph), "hipGraphDestroy")
+    for a in (u, r):
+        a.free()
+    s.destroy()
