@@ -427,8 +427,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
     }
   };
   if (kEarly && longest > 0) entries(0);
-  W5<C> wc{};
-  if (kEarly && inside) wc = load_w(d.prim, c);
+  W5<C> wc = kEarly && inside ? load_w(d.prim, c) : W5<C>{};
   for (int j = threadIdx.x; j < tn; j += kBlock) {
     const int e = d.tent[t0 + j];
     const W5<C> w = e >= 0 ? load_w(d.prim, e) : load_w(d.prim_b, -e - 1);
