@@ -1405,7 +1405,7 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(OCC > 0 
 // so bound by the chain of its loads: each wave takes nslot / 16 slots and has all their words in
 // flight, then adds them into LDS; the rest is the face blocks' keys, whose number grows with the mesh. With
 // one thread per word adding 64 slots in turn this took 17 us of a step of 33k cells, now 5.3; 28 of 796k
-// tetrahedra, now 8.8; 32 of a 2.3M-cell channel, now 10; 43 of 7.9M cells, now 15.7.
+// tetrahedra, now 8.8; 32 of a 2.3M-cell channel, now 10; 43 of 7.9M cells, now 14.
 __global__ __launch_bounds__(1024) void k_step_reduce(const long long* __restrict__ nslots, int nslot,
                                                       const unsigned long long* __restrict__ partial,
                                                       const int* __restrict__ fcbeg, const int* __restrict__ cflags,
