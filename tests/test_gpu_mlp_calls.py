@@ -62,10 +62,13 @@ def test_layered_prediction_holds_a_chunk_of_activations(hidden, fused):
 def test_a_wide_network_holds_no_operand_packs():
     """Networks wider than the fused kernels hold, per parameter, the FP32 weight, gradient and Adam's
     two moments, the BF16 weight and a mask byte: nothing laid out for kernels that they never run."""
+    small = MLP(7, 64, 1, 5)  # what a process's first network makes the runtime allocate
+    small.predict(samples(10, 1))
     before = free_bytes()
     m = MLP(7, 2048, 4, 5, seed=4)
     assert before - free_bytes() <= m.param_count * (4 * 4 + 2 + 1) + (32 << 20)
     m.close()
+    small.close()
 
 
 def test_data_that_does_not_fit_leaves_none():
